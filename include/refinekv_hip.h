@@ -77,6 +77,25 @@ int rkv_summary_store(const void* keys, int64_t k_head_stride, int64_t k_token_s
                       int64_t* counts, void* key_mean, void* value_mean, void* ellipsoid,
                       float* value_norm, float* max_value_norm, rkv_stream_t stream);
 
+/*
+ * rkv_summary that also writes the pages the summary holds -- the prompt in
+ * whole blocks, (heads, ceil(length / block_size) * block_size, dim) dense,
+ * rows past the prompt's end zero -- from the same read of keys / values, and
+ * the cache as rkv_summary_store does when cache_keys and cache_values are
+ * given (NULL, NULL: no cache).  Replaces the padded copy of
+ * src/refinekv/summary.py:35-43, which a prompt that is not whole blocks, or
+ * whose rows are not dense, needs.  key_pages or value_pages may be NULL (that
+ * tensor's pages view the cache).
+ */
+int rkv_summary_pages(const void* keys, int64_t k_head_stride, int64_t k_token_stride,
+                      const void* values, int64_t v_head_stride, int64_t v_token_stride,
+                      int dtype, int64_t heads, int64_t length, int64_t dim, int64_t block_size,
+                      void* cache_keys, int64_t ck_head_stride, int64_t ck_token_stride,
+                      void* cache_values, int64_t cv_head_stride, int64_t cv_token_stride,
+                      void* key_pages, void* value_pages, int64_t* counts, void* key_mean,
+                      void* value_mean, void* ellipsoid, float* value_norm,
+                      float* max_value_norm, rkv_stream_t stream);
+
 /* Workspace bytes needed by rkv_select / rkv_decode for this shape (device
  * memory the caller owns).  Zero-fill it when it is created: its first region
  * holds rkv_decode's hand-off counters, which count this shape's tiles (each

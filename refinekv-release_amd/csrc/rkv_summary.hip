@@ -180,15 +180,25 @@ __host__ __device__ constexpr int64_t summary_wave_lds(bool stage, int64_t dim, 
   return (stage ? 2 * block * dim * elem : 0) + 2 * dim * 4;
 }
 
-// Where the keys and values also go when the summary is built while the
-// prompt is written to the cache (kStore): the same element strides as the
-// sources' meaning (head, token), head_dim dense.
+// A place the keys and values also go while the summary reads them: element
+// strides as the sources' (head, token), head_dim dense.  A null tensor is
+// not written.  pad: rows past the prompt's end up to the whole block are
+// written too, as zeros.  wide: every row starts on a 16-byte boundary.
 template <class In>
-struct CacheOut {
+struct RowsOut {
   typename In::T* keys;
   int64_t k_hs, k_ts;
   typename In::T* values;
   int64_t v_hs, v_ts;
+  bool pad, wide;
+};
+
+// The places a kernel with kStore of them writes: the KV cache, the
+// summary's zero-padded pages, or both in this order.
+template <class In>
+struct CacheOut {
+  RowsOut<In> to[2];
+  int n;
 };
 
 // Byte strides of a block's rows fit 31 bits (checked on the host).
@@ -209,7 +219,7 @@ struct SplitPart {
   float* part;      // LDS: waves x 4 x D floats (chunk sums, max, min), then waves x 2
 };
 
-template <int D, class In, bool kStore, bool kStage, bool kSplit = false>
+template <int D, class In, int kStore, bool kStage, bool kSplit = false>
 __device__ __forceinline__ void summary_passes(
     int64_t h, int64_t b, int64_t row0, bool valid, int cnt, int block, int64_t n_blocks,
     __amdgpu_buffer_rsrc_t kr, __amdgpu_buffer_rsrc_t vr, int kts, int vts, const uint4* kst,
@@ -296,21 +306,70 @@ __device__ __forceinline__ void summary_passes(
     kmax[j] = kNegInf;
     kmin[j] = kPosInf;
   }
-  // the cache rows of this block (kStore): live tokens, lanes on1
-  const int cks = kStore ? (int)out.k_ts * E : 0, cvs = kStore ? (int)out.v_ts * E : 0;
-  const auto ckr =
-      kStore ? rows_view(out.keys + h * out.k_hs + row0 * out.k_ts, extent(cks)) : kr;
-  const auto cvr =
-      kStore ? rows_view(out.values + h * out.v_hs + row0 * out.v_ts, extent(cvs)) : vr;
+  // The rows of this block in each place they go to (kStore): views that
+  // end with the live tokens, or with the whole block where it is padded
+  // (stores past a view's end are dropped).
+  // Staged rows of 2-byte elements up to head_dim 128 go out as they came in,
+  // 16 bytes per lane from LDS (rows past the live tokens were read as
+  // zeros), where pass 1's registers hold 4 bytes per lane: a quarter of the
+  // store instructions (prompt of 8 heads x 32768 tokens, d 128, B 32,
+  // written to the cache: 60.6 -> 57.7 us).  Elsewhere a lane's registers hold
+  // 8 bytes or more and the extra LDS reads do not pay (fp32 109.8 -> 110.4,
+  // d 256 B 16 125.3 -> 127.1).
+  constexpr bool kWide = kStage && E * CPL == 4;
+  struct Dest {
+    __amdgpu_buffer_rsrc_t k, v;
+    int ks, vs;
+    bool narrow;
+  };
+  auto dest = [&](int i) {
+    const RowsOut<In>& o = out.to[i];
+    Dest d;
+    d.ks = (int)o.k_ts * E;
+    d.vs = (int)o.v_ts * E;
+    const int rows = o.pad ? (valid ? block : 0) : cnt;
+    auto bytes = [&](const T* p, int ts) {
+      return __builtin_amdgcn_readfirstlane(p && rows ? (rows - 1) * ts + D * E : 0);
+    };
+    d.k = rows_view(o.keys + h * o.k_hs + row0 * o.k_ts, bytes(o.keys, d.ks));
+    d.v = rows_view(o.values + h * o.v_hs + row0 * o.v_ts, bytes(o.values, d.vs));
+    d.narrow = !kWide || !o.wide;
+    return d;
+  };
+  Dest dst[kStore > 0 ? kStore : 1];
+  if constexpr (kStore > 0) {
+#pragma unroll
+    for (int i = 0; i < kStore; ++i) dst[i] = dest(i);
+    if constexpr (kWide) {
+      for (int p0 = 0; p0 < block * St::NC; p0 += kWave) {
+        const int p = p0 + lane, t = p / St::NC;
+        const int off = St::slot(p % St::NC, t) * 16;
+        typedef unsigned int U4 __attribute__((ext_vector_type(4)));
+        const U4 kq = __builtin_bit_cast(U4, kst[p]), vq = __builtin_bit_cast(U4, vst[p]);
+#pragma unroll
+        for (int i = 0; i < kStore; ++i) {
+          if (dst[i].narrow) continue;
+          __builtin_amdgcn_raw_buffer_store_b128(kq, dst[i].k, t * dst[i].ks + off, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b128(vq, dst[i].v, t * dst[i].vs + off, 0, 0);
+        }
+      }
+    }
+  }
+  auto store = [&](int t, const RawCols<In, CPL>& rk, const RawCols<In, CPL>& rv) {
+    if constexpr (kStore > 0) {
+#pragma unroll
+      for (int i = 0; i < kStore; ++i) {
+        if (on1 && dst[i].narrow) {
+          buf_store_cols<In, CPL>(dst[i].k, col * E, t * dst[i].ks, rk);
+          buf_store_cols<In, CPL>(dst[i].v, col * E, t * dst[i].vs, rv);
+        }
+      }
+    }
+  };
   // token t's columns added to the chunk sums (t < cnt, wave-uniform)
   auto take = [&](int t, const RawCols<In, CPL>& rk, const RawCols<In, CPL>& rv,
                   float (&ak)[CPL], float (&av)[CPL], float (&xk)[CPL]) {
-    if constexpr (kStore) {
-      if (on1) {
-        buf_store_cols<In, CPL>(ckr, col * E, t * cks, rk);
-        buf_store_cols<In, CPL>(cvr, col * E, t * cvs, rv);
-      }
-    }
+    store(t, rk, rv);
     float xv[CPL];
     cols_f32<In, CPL>(rk, xk);
     cols_f32<In, CPL>(rv, xv);
@@ -362,6 +421,10 @@ __device__ __forceinline__ void summary_passes(
           kmax[j] = max3_nan(kmax[j], x[j], x[j]);
           kmin[j] = min3_nan(kmin[j], x[j], x[j]);
         }
+      }
+      if constexpr (kStore > 0) {
+        const RawCols<In, CPL> zero = {};
+        for (int t = cnt > c0 ? cnt : c0; t < c0 + 16; ++t) store(t, zero, zero);
       }
       // the chunk's padded tokens each add +0, as the reference's zero-padded
       // pages do (repeated +0 adds equal one)
@@ -570,7 +633,7 @@ __device__ __forceinline__ void summary_passes(
   }
 }
 
-template <int D, class In, bool kStore, bool kStage>
+template <int D, class In, int kStore, bool kStage>
 __global__ __launch_bounds__(kWave * kSummaryWaves) void summary_kernel(
     const typename In::T* __restrict__ keys, int64_t k_hs, int64_t k_ts,
     const typename In::T* __restrict__ values, int64_t v_hs, int64_t v_ts, int64_t length,
@@ -627,7 +690,7 @@ __global__ __launch_bounds__(kWave * kSummaryWaves) void summary_kernel(
 // kSplit), so HBM sees each row once.  LDS: the waves' chunks (K then V, the
 // staged layout), then D key means, D inverse widths and the chunks'
 // partials.
-template <int D, class In, bool kStore>
+template <int D, class In, int kStore>
 __global__ __launch_bounds__(kWave * 4) void summary_split_kernel(
     const typename In::T* __restrict__ keys, int64_t k_hs, int64_t k_ts,
     const typename In::T* __restrict__ values, int64_t v_hs, int64_t v_ts, int64_t length,
@@ -683,7 +746,7 @@ constexpr int64_t summary_split_lds(int64_t dim, int64_t elem, int64_t block) {
 // computes with none in flight.  The passes are summary_kernel's.
 constexpr int kStreamChunks = 8;  // 16-byte chunks per lane per tensor, at most
 
-template <int D, class In, bool kStore>
+template <int D, class In, int kStore>
 __global__ __launch_bounds__(kWave) void summary_stream_kernel(
     const typename In::T* __restrict__ keys, int64_t k_hs, int64_t k_ts,
     const typename In::T* __restrict__ values, int64_t v_hs, int64_t v_ts, int64_t length,
@@ -824,8 +887,9 @@ int launch_summary(const void* keys, int64_t k_hs, int64_t k_ts, const void* val
           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) ==
               hipSuccess &&
           hipOccupancyMaxActiveBlocksPerMultiprocessor(
-              &per_cu, out.keys ? summary_stream_kernel<D, In, true>
-                                : summary_stream_kernel<D, In, false>,
+              &per_cu, out.n == 2   ? summary_stream_kernel<D, In, 2>
+                       : out.n == 1 ? summary_stream_kernel<D, In, 1>
+                                    : summary_stream_kernel<D, In, 0>,
               kWave, (size_t)per_wave) == hipSuccess)
         resident = (int64_t)cus * per_cu;
     });
@@ -833,20 +897,22 @@ int launch_summary(const void* keys, int64_t k_hs, int64_t k_ts, const void* val
     const int64_t grid = resident > 0 ? (resident < total ? resident : total) : total;
     const auto* k = static_cast<const typename In::T*>(keys);
     const auto* v = static_cast<const typename In::T*>(values);
-    RKV_DISPATCH_DIM(dim, D, {
-      if (out.keys)
-        summary_stream_kernel<D, In, true><<<dim3((unsigned)grid), dim3(kWave), per_wave,
-                                              stream>>>(
-            k, k_hs, k_ts, v, v_hs, v_ts, length, (int)block, n_blocks, heads, counts,
-            static_cast<uint16_t*>(key_mean), static_cast<uint16_t*>(value_mean),
-            static_cast<uint16_t*>(ellipsoid), value_norm, out);
-      else
-        summary_stream_kernel<D, In, false><<<dim3((unsigned)grid), dim3(kWave), per_wave,
-                                               stream>>>(
-            k, k_hs, k_ts, v, v_hs, v_ts, length, (int)block, n_blocks, heads, counts,
-            static_cast<uint16_t*>(key_mean), static_cast<uint16_t*>(value_mean),
-            static_cast<uint16_t*>(ellipsoid), value_norm, out);
-    });
+#define RKV_SUMMARY_LAUNCH(STORE)                                                              \
+  RKV_DISPATCH_DIM(dim, D,                                                                     \
+                   summary_stream_kernel<D, In, STORE>                                         \
+                   <<<dim3((unsigned)grid), dim3(kWave), per_wave, stream>>>(                  \
+                       k, k_hs, k_ts, v, v_hs, v_ts, length, (int)block, n_blocks, heads,      \
+                       counts, static_cast<uint16_t*>(key_mean),                               \
+                       static_cast<uint16_t*>(value_mean), static_cast<uint16_t*>(ellipsoid),  \
+                       value_norm, out))
+    if (out.n == 2) {
+      RKV_SUMMARY_LAUNCH(2);
+    } else if (out.n == 1) {
+      RKV_SUMMARY_LAUNCH(1);
+    } else {
+      RKV_SUMMARY_LAUNCH(0);
+    }
+#undef RKV_SUMMARY_LAUNCH
     int rc = check_launch("summary_stream_kernel");
     if (rc) return rc;
     max_norm_kernel<<<dim3((unsigned)heads), dim3(256), 0, stream>>>(value_norm, n_blocks,
@@ -869,16 +935,20 @@ int launch_summary(const void* keys, int64_t k_hs, int64_t k_ts, const void* val
       rows16(keys, k_hs, k_ts) && rows16(values, v_hs, v_ts)) {
     const dim3 sgrid((unsigned)n_blocks, (unsigned)heads);
     const dim3 sthreads((unsigned)(kWave * (block / 16)));
-    RKV_DISPATCH_DIM(dim, D, {
-      if (out.keys)
-        summary_split_kernel<D, In, true><<<sgrid, sthreads, (size_t)split_lds, stream>>>(
-            k, k_hs, k_ts, v, v_hs, v_ts, length, (int)block, n_blocks, counts, km, vm, el,
-            value_norm, out);
-      else
-        summary_split_kernel<D, In, false><<<sgrid, sthreads, (size_t)split_lds, stream>>>(
-            k, k_hs, k_ts, v, v_hs, v_ts, length, (int)block, n_blocks, counts, km, vm, el,
-            value_norm, out);
-    });
+#define RKV_SUMMARY_LAUNCH(STORE)                                                            \
+  RKV_DISPATCH_DIM(dim, D,                                                                   \
+                   summary_split_kernel<D, In, STORE>                                        \
+                   <<<sgrid, sthreads, (size_t)split_lds, stream>>>(                         \
+                       k, k_hs, k_ts, v, v_hs, v_ts, length, (int)block, n_blocks, counts,   \
+                       km, vm, el, value_norm, out))
+    if (out.n == 2) {
+      RKV_SUMMARY_LAUNCH(2);
+    } else if (out.n == 1) {
+      RKV_SUMMARY_LAUNCH(1);
+    } else {
+      RKV_SUMMARY_LAUNCH(0);
+    }
+#undef RKV_SUMMARY_LAUNCH
     int rc = check_launch("summary_split_kernel");
     if (rc) return rc;
     max_norm_kernel<<<dim3((unsigned)heads), dim3(256), 0, stream>>>(value_norm, n_blocks,
@@ -895,14 +965,18 @@ int launch_summary(const void* keys, int64_t k_hs, int64_t k_ts, const void* val
                    summary_kernel<D, In, STORE, STAGE><<<grid, threads, lds, stream>>>(    \
                        k, k_hs, k_ts, v, v_hs, v_ts, length, (int)block, n_blocks, counts, \
                        km, vm, el, value_norm, out))
-  if (out.keys && stage) {
-    RKV_SUMMARY_LAUNCH(true, true);
-  } else if (out.keys) {
-    RKV_SUMMARY_LAUNCH(true, false);
+  if (out.n == 2 && stage) {
+    RKV_SUMMARY_LAUNCH(2, true);
+  } else if (out.n == 2) {
+    RKV_SUMMARY_LAUNCH(2, false);
+  } else if (out.n == 1 && stage) {
+    RKV_SUMMARY_LAUNCH(1, true);
+  } else if (out.n == 1) {
+    RKV_SUMMARY_LAUNCH(1, false);
   } else if (stage) {
-    RKV_SUMMARY_LAUNCH(false, true);
+    RKV_SUMMARY_LAUNCH(0, true);
   } else {
-    RKV_SUMMARY_LAUNCH(false, false);
+    RKV_SUMMARY_LAUNCH(0, false);
   }
 #undef RKV_SUMMARY_LAUNCH
   int rc = check_launch("summary_kernel");
@@ -924,8 +998,9 @@ int summary_impl(const char* who, const void* keys, int64_t k_head_stride,
                  int64_t v_token_stride, int dtype, int64_t heads, int64_t length, int64_t dim,
                  int64_t block_size, void* cache_keys, int64_t ck_head_stride,
                  int64_t ck_token_stride, void* cache_values, int64_t cv_head_stride,
-                 int64_t cv_token_stride, int64_t* counts, void* key_mean, void* value_mean,
-                 void* ellipsoid, float* value_norm, float* max_value_norm, hipStream_t stream) {
+                 int64_t cv_token_stride, void* key_pages, void* value_pages, int64_t* counts,
+                 void* key_mean, void* value_mean, void* ellipsoid, float* value_norm,
+                 float* max_value_norm, hipStream_t stream) {
   if (!keys || !values || !counts || !key_mean || !value_mean || !ellipsoid || !value_norm ||
       !max_value_norm)
     return set_error(kInvalidArgument, "%s: null pointer argument", who);
@@ -970,35 +1045,31 @@ int summary_impl(const char* who, const void* keys, int64_t k_head_stride,
       (store && (ck_token_stride >= row_limit || cv_token_stride >= row_limit)))
     return set_error(kUnsupported, "%s: token stride above %lld elements", who,
                      (long long)(row_limit - 1));
-  switch (dtype) {
-    case 0: {
-      const CacheOut<InBf16> out{static_cast<uint16_t*>(cache_keys), ck_head_stride,
-                                 ck_token_stride, static_cast<uint16_t*>(cache_values),
-                                 cv_head_stride, cv_token_stride};
-      return launch_summary<InBf16>(keys, k_head_stride, k_token_stride, values, v_head_stride,
-                                    v_token_stride, heads, length, dim, block_size, counts,
-                                    key_mean, value_mean, ellipsoid, value_norm, max_value_norm,
-                                    out, stream);
-    }
-    case 1: {
-      const CacheOut<InF16> out{static_cast<uint16_t*>(cache_keys), ck_head_stride,
-                                ck_token_stride, static_cast<uint16_t*>(cache_values),
-                                cv_head_stride, cv_token_stride};
-      return launch_summary<InF16>(keys, k_head_stride, k_token_stride, values, v_head_stride,
-                                   v_token_stride, heads, length, dim, block_size, counts,
-                                   key_mean, value_mean, ellipsoid, value_norm, max_value_norm,
-                                   out, stream);
-    }
-    default: {
-      const CacheOut<InF32> out{static_cast<float*>(cache_keys), ck_head_stride, ck_token_stride,
-                                static_cast<float*>(cache_values), cv_head_stride,
-                                cv_token_stride};
-      return launch_summary<InF32>(keys, k_head_stride, k_token_stride, values, v_head_stride,
-                                   v_token_stride, heads, length, dim, block_size, counts,
-                                   key_mean, value_mean, ellipsoid, value_norm, max_value_norm,
-                                   out, stream);
-    }
-  }
+  if (!aligned(key_pages, need) || !aligned(value_pages, need))
+    return set_error(kInvalidArgument, "%s: pages must be %d-byte aligned", who, (int)need);
+  auto launch = [&](auto in) {
+    using In = decltype(in);
+    using T = typename In::T;
+    CacheOut<In> out{};
+    auto add = [&](void* k, int64_t k_hs, int64_t k_ts, void* v, int64_t v_hs, int64_t v_ts,
+                   bool pad) {
+      const int64_t strides = (k_hs | k_ts | v_hs | v_ts) * elem;
+      out.to[out.n++] = RowsOut<In>{static_cast<T*>(k), k_hs, k_ts, static_cast<T*>(v), v_hs, v_ts,
+                                    pad, strides % 16 == 0 && aligned(k, 16) && aligned(v, 16)};
+    };
+    if (store)
+      add(cache_keys, ck_head_stride, ck_token_stride, cache_values, cv_head_stride,
+          cv_token_stride, false);
+    if (key_pages || value_pages)
+      add(key_pages, n_blocks * block_size * dim, dim, value_pages, n_blocks * block_size * dim,
+          dim, true);
+    return launch_summary<In>(keys, k_head_stride, k_token_stride, values, v_head_stride,
+                              v_token_stride, heads, length, dim, block_size, counts, key_mean,
+                              value_mean, ellipsoid, value_norm, max_value_norm, out, stream);
+  };
+  if (dtype == 0) return launch(InBf16{});
+  if (dtype == 1) return launch(InF16{});
+  return launch(InF32{});
 }
 
 }  // namespace
@@ -1012,8 +1083,8 @@ extern "C" int rkv_summary(const void* keys, int64_t k_head_stride, int64_t k_to
   clear_error();
   return summary_impl("rkv_summary", keys, k_head_stride, k_token_stride, values, v_head_stride,
                       v_token_stride, dtype, heads, length, dim, block_size, nullptr, 0, 0,
-                      nullptr, 0, 0, counts, key_mean, value_mean, ellipsoid, value_norm,
-                      max_value_norm, stream);
+                      nullptr, 0, 0, nullptr, nullptr, counts, key_mean, value_mean, ellipsoid,
+                      value_norm, max_value_norm, stream);
 }
 
 extern "C" int rkv_summary_store(const void* keys, int64_t k_head_stride,
@@ -1032,6 +1103,24 @@ extern "C" int rkv_summary_store(const void* keys, int64_t k_head_stride,
   return summary_impl("rkv_summary_store", keys, k_head_stride, k_token_stride, values,
                       v_head_stride, v_token_stride, dtype, heads, length, dim, block_size,
                       cache_keys, ck_head_stride, ck_token_stride, cache_values, cv_head_stride,
-                      cv_token_stride, counts, key_mean, value_mean, ellipsoid, value_norm,
+                      cv_token_stride, nullptr, nullptr, counts, key_mean, value_mean, ellipsoid, value_norm,
                       max_value_norm, stream);
+}
+
+extern "C" int rkv_summary_pages(const void* keys, int64_t k_head_stride,
+                                 int64_t k_token_stride, const void* values,
+                                 int64_t v_head_stride, int64_t v_token_stride, int dtype,
+                                 int64_t heads, int64_t length, int64_t dim, int64_t block_size,
+                                 void* cache_keys, int64_t ck_head_stride,
+                                 int64_t ck_token_stride, void* cache_values,
+                                 int64_t cv_head_stride, int64_t cv_token_stride,
+                                 void* key_pages, void* value_pages, int64_t* counts,
+                                 void* key_mean, void* value_mean, void* ellipsoid,
+                                 float* value_norm, float* max_value_norm, hipStream_t stream) {
+  clear_error();
+  return summary_impl("rkv_summary_pages", keys, k_head_stride, k_token_stride, values,
+                      v_head_stride, v_token_stride, dtype, heads, length, dim, block_size,
+                      cache_keys, ck_head_stride, ck_token_stride, cache_values, cv_head_stride,
+                      cv_token_stride, key_pages, value_pages, counts, key_mean, value_mean,
+                      ellipsoid, value_norm, max_value_norm, stream);
 }

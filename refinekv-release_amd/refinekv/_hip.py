@@ -53,6 +53,9 @@ def _bind(lib):
                                       _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p,
                                       _p, _p]
     lib.rkv_summary_store.restype = _int
+    lib.rkv_summary_pages.argtypes = (lib.rkv_summary_store.argtypes[:-7] + [_p, _p]
+                                      + lib.rkv_summary_store.argtypes[-7:])
+    lib.rkv_summary_pages.restype = _int
     lib.rkv_workspace_bytes.argtypes = [_i64, _i64, _i64, _i64]
     lib.rkv_workspace_bytes.restype = _size
     lib.rkv_workspace_layout.argtypes = [_i64, _i64, _i64, _i64, _p]
@@ -145,11 +148,14 @@ def _row_aligned(t, nbytes):
     return t if ok else t.clone(memory_format=torch.contiguous_format)
 
 
-def summary_fields(keys, values, block, cache_keys=None, cache_values=None):
+def summary_fields(keys, values, block, cache_keys=None, cache_values=None, key_pages=None,
+                   value_pages=None):
     """Run the summary kernel on (H, L, D) keys/values; returns the tensors of
     BlockSummary other than the page views.  With cache_keys / cache_values
     ((H, L, D) views of the KV cache, head_dim dense) the same kernel also
-    writes every token there (rkv_summary_store)."""
+    writes every token there, and with key_pages / value_pages (contiguous
+    (H, N, B, D), either alone or both) the zero-padded pages
+    (rkv_summary_pages)."""
     heads, length, dim = keys.shape
     need = keys.element_size() * (2 if dim <= 128 else 4)
     keys, values = _row_aligned(keys, need), _row_aligned(values, need)
@@ -166,16 +172,19 @@ def summary_fields(keys, values, block, cache_keys=None, cache_values=None):
     sources = (_ptr(keys), keys.stride(0), keys.stride(1), _ptr(values), values.stride(0),
                values.stride(1), DTYPE_CODES[keys.dtype], heads, length, dim, block)
     if cache_keys is None:
+        cache = (None, 0, 0, None, 0, 0)
+    else:
+        for view in (cache_keys, cache_values):
+            if (view.shape != keys.shape or view.dtype != keys.dtype or view.stride(-1) != 1
+                    or view.device != dev):
+                raise ValueError("cache views must match keys/values with a dense head_dim")
+        cache = (_ptr(cache_keys), cache_keys.stride(0), cache_keys.stride(1),
+                 _ptr(cache_values), cache_values.stride(0), cache_values.stride(1))
+    if cache_keys is None and key_pages is None and value_pages is None:
         _check(lib().rkv_summary(*sources, *outputs), "rkv_summary")
     else:
-        for cache in (cache_keys, cache_values):
-            if (cache.shape != keys.shape or cache.dtype != keys.dtype or cache.stride(-1) != 1
-                    or cache.device != dev):
-                raise ValueError("cache views must match keys/values with a dense head_dim")
-        rc = lib().rkv_summary_store(
-            *sources, _ptr(cache_keys), cache_keys.stride(0), cache_keys.stride(1),
-            _ptr(cache_values), cache_values.stride(0), cache_values.stride(1), *outputs)
-        _check(rc, "rkv_summary_store")
+        _check(lib().rkv_summary_pages(*sources, *cache, _ptr(key_pages), _ptr(value_pages),
+                                       *outputs), "rkv_summary_pages")
     return counts, key_mean, value_mean, ellipsoid, value_norm, max_value_norm
 
 
