@@ -147,8 +147,8 @@ int rkv_select(const void* query, const void* key_mean, const void* ellipsoid,
  * Prompt-anchor mask: the union of the expanded-block masks of `anchors`
  * queries.  Replaces the per-anchor loop of select_blocks calls in the
  * reference's Transformers hook (src/refinekv/integrations/
- * transformers.py:539-552) with one scoring launch over every (query, head,
- * tile) and one launch that ORs the decisions.
+ * transformers.py:539-552) with one scoring launch over every query row and
+ * tile, one that merges the rows' log Z / log C and one that decides and ORs.
  *   queries: (anchors, heads, group, dim) bf16, dense.  Summary and eps /
  *   reduction as for rkv_select (each query is reduced over its own group).
  *   mask_out: (heads, n_blocks) bytes 0/1.
@@ -162,6 +162,19 @@ int rkv_select_anchors(const void* queries, const void* key_mean, const void* el
                        int64_t prompt_length, float eps, int reduction, int64_t anchors,
                        uint8_t* mask_out, void* workspace, size_t workspace_bytes,
                        rkv_stream_t stream);
+
+/* rkv_select_anchors for queries in any order of axes: query row (anchor,
+ * head, g) starts q_anchor_stride, q_head_stride and q_row_stride elements
+ * (multiples of 8) apart, dim dense, e.g. the (heads, group, anchors, dim)
+ * rows of a projection. */
+int rkv_select_anchors_strided(const void* queries, int64_t q_anchor_stride,
+                               int64_t q_head_stride, int64_t q_row_stride, const void* key_mean,
+                               const void* ellipsoid, const float* value_norm,
+                               const float* max_value_norm, int64_t heads, int64_t group,
+                               int64_t dim, int64_t n_blocks, int64_t block_size,
+                               int64_t prompt_length, float eps, int reduction, int64_t anchors,
+                               uint8_t* mask_out, void* workspace, size_t workspace_bytes,
+                               rkv_stream_t stream);
 
 /*
  * One decode step of RefineKV attention.  Replaces sparse_attention_triton

@@ -45,6 +45,7 @@
 // Every order is fixed, so masks and outputs are deterministic run to run.
 #include <math.h>
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 #include <utility>
@@ -524,11 +525,11 @@ __device__ __forceinline__ void score_dots(const ScoreArgs& a, int64_t h, int64_
 // z, delta, the risk's delta-only factors and the tile's LSE partials from
 // the dot products: wave w owns rows w, w + 4, ...; lane = block of the
 // tile.  put_z(g, valid, (z, delta, A, th)) is called by every lane (valid:
-// the block exists); put_lse(g, (zm, zl, cm, cl)) by lane 0.
+// the block exists); put_lse(g, (zm, zl, cm, cl)) by lane 0.  G rows.
 template <typename PutZ, typename PutLse>
-__device__ __forceinline__ void score_stats(const ScoreArgs& a, int64_t tile, const float* sdot,
-                                            const float* pdot, PutZ put_z, PutLse put_lse) {
-  const int G = a.group;
+__device__ __forceinline__ void score_stats(const ScoreArgs& a, int G, int64_t tile,
+                                            const float* sdot, const float* pdot, PutZ put_z,
+                                            PutLse put_lse) {
   const int64_t N = a.n_blocks;
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // wave-uniform
@@ -566,7 +567,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   const int lane = threadIdx.x % kWave;
   score_dots<D, kMaxGroup, true>(a, h, tile, sdot, pdot, pdot + G * kTile);
   score_stats(
-      a, tile, sdot, pdot,
+      a, G, tile, sdot, pdot,
       [&](int g, bool valid, float4 zf) {
         if (valid) a.zf[(h * G + g) * a.z_stride + tile * kTile + lane] = zf;
       },
@@ -648,12 +649,9 @@ struct DecideLoads {
 
 // kStats = false leaves part and zf to the caller (the one-launch step has
 // them only after its hand-off).
-// rh: the head index of the statistics rows (lse, zf) -- h except for the
-// batched anchor selection, whose query q of head h has rows of head q H + h.
 template <bool kStats = true>
 __device__ __forceinline__ DecideLoads decide_issue(const DecideArgs& a, int64_t h,
-                                                    int64_t tile, int64_t rh = -1) {
-  if (rh < 0) rh = h;
+                                                    int64_t tile) {
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // wave-uniform
   const int G = a.group;
@@ -667,8 +665,8 @@ __device__ __forceinline__ DecideLoads decide_issue(const DecideArgs& a, int64_t
   d.vnorm = a.value_norm[h * N + bc];
   d.anc = anc[h * N + bc];
   if constexpr (kStats) {
-    d.part = *reinterpret_cast<const float4*>(a.lse + ((rh * G + gl) * a.tile_stride + tl) * 4);
-    d.zf = a.zf[(rh * G + gl) * a.z_stride + bc];
+    d.part = *reinterpret_cast<const float4*>(a.lse + ((h * G + gl) * a.tile_stride + tl) * 4);
+    d.zf = a.zf[(h * G + gl) * a.z_stride + bc];
   }
   return d;
 }
@@ -939,9 +937,7 @@ __device__ __forceinline__ uint64_t decide_finish(const DecideArgs& a, int64_t h
                                                   const DecideLoads& in, DecideShared& sh,
                                                   float (*zsh)[kTile], const int32_t*& list,
                                                   uint32_t& count,
-                                                  const StepStats* ss = nullptr,
-                                                  int64_t rh = -1) {
-  if (rh < 0) rh = h;
+                                                  const StepStats* ss = nullptr) {
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // wave-uniform
   const int G = a.group;
@@ -960,14 +956,14 @@ __device__ __forceinline__ uint64_t decide_finish(const DecideArgs& a, int64_t h
   bool wbad = false;
   auto row_tail = [&](int g, float lz, float lc, float4 zf) {
     if (a.stats_out && owner && tile == 0 && lane == 0) {
-      a.stats_out[(rh * G + g) * 2] = lz;
-      a.stats_out[(rh * G + g) * 2 + 1] = lc;
+      a.stats_out[(h * G + g) * 2] = lz;
+      a.stats_out[(h * G + g) * 2 + 1] = lc;
     }
     wbad |= !is_finite(lz) || !is_finite(lc);
     float r = 0.0f;
     if (valid) {
       r = risk_from(zf.x, zf.y, zf.z, zf.w, lz, lc, vmax, vnorm);
-      if (a.risk_out && owner) a.risk_out[(rh * G + g) * N + b] = r;
+      if (a.risk_out && owner) a.risk_out[(h * G + g) * N + b] = r;
     }
     wsel |= __ballot(valid && (r > a.eps || !is_finite(r)));
     sh.risk[g][lane] = r;
@@ -1002,10 +998,10 @@ __device__ __forceinline__ uint64_t decide_finish(const DecideArgs& a, int64_t h
     auto row_stats = [&](int g, float4 part, float4 zf) {
       if (a.row_lse != nullptr) {
         // (merged once per row by lse_merge_kernel, in this same order)
-        row_tail(g, a.row_lse[(rh * G + g) * 2], a.row_lse[(rh * G + g) * 2 + 1], zf);
+        row_tail(g, a.row_lse[(h * G + g) * 2], a.row_lse[(h * G + g) * 2 + 1], zf);
         return;
       }
-      const float* prow = a.lse + (rh * G + g) * a.tile_stride * 4;
+      const float* prow = a.lse + (h * G + g) * a.tile_stride * 4;
       if (lane >= T) part = make_float4(kNegInf, 0.0f, kNegInf, 0.0f);
       auto pz = [&](int64_t t) { return make_float2(prow[t * 4], prow[t * 4 + 1]); };
       auto pc = [&](int64_t t) { return make_float2(prow[t * 4 + 2], prow[t * 4 + 3]); };
@@ -1017,9 +1013,9 @@ __device__ __forceinline__ uint64_t decide_finish(const DecideArgs& a, int64_t h
     if (wave < G) row_stats(wave, in.part, in.zf);
 #pragma unroll 1
     for (int g = wave + kWaves; g < G; g += kWaves) {
-      const int64_t at = (rh * G + g) * a.tile_stride + tl;
+      const int64_t at = (h * G + g) * a.tile_stride + tl;
       row_stats(g, *reinterpret_cast<const float4*>(a.lse + at * 4),
-                a.zf[(rh * G + g) * a.z_stride + bc]);
+                a.zf[(h * G + g) * a.z_stride + bc]);
     }
   }
   if (lane == 0) {
@@ -1219,25 +1215,230 @@ __global__ __launch_bounds__(kThreads) void lse_merge_kernel(const float* lse, f
   }
 }
 
-// Batched anchor selection: the union over `anchors` queries of their
-// decisions, for tile (blockIdx.x) of head h (blockIdx.y); query q's rows are
-// those of head q H + h.  The OR of the tiles' ballots is stored once.
-__global__ __launch_bounds__(kThreads) void anchor_decide_kernel(DecideArgs a, int anchors,
-                                                                 int heads, uint8_t* mask_out) {
-  __shared__ DecideShared sh;
-  const int64_t h = blockIdx.y, tile = blockIdx.x;
-  uint64_t any = 0;
-  for (int q = 0; q < anchors; ++q) {
-    const int64_t rh = (int64_t)q * heads + h;
-    const DecideLoads in = decide_issue(a, h, tile, rh);
-    const int32_t* list;
-    uint32_t count = 0;
-    any |= decide_finish(a, h, tile, in, sh, nullptr, list, count, nullptr, rh);
-    __syncthreads();  // the next query reuses sh
+// ---------------------------------------------------------------------------
+// Batched anchor selection: the union over many queries of their decisions
+// ---------------------------------------------------------------------------
+// Three launches: anchor_rows_kernel (the score phase of every query row),
+// lse_merge_kernel (each row's log Z / log C), anchor_decide_kernel (risks,
+// reduction and the union).  A head's query rows are one list, row r = anchor
+// r / G, query head r % G; the statistics of row r of head h sit at
+// workspace row h R + r, R = anchors x G.
+struct AnchorArgs {
+  ScoreArgs score;
+  const float* row_lse;         // (H R, 2): log Z, log C
+  const float* value_norm;      // (H, N)
+  const float* max_value_norm;  // (H)
+  uint8_t* mask;                // (H, N)
+  int64_t q_as, q_hs, q_gs;     // query strides (elements): anchor, head, group row
+  int rows, per;                // R; rows (anchor_decide_kernel: anchors) per workgroup
+  int anchors, n_tiles, reduction;
+  float eps;
+};
+
+// Scores of rows [z per, (z + 1) per) of head h against tile `tile`, blockIdx
+// (tile, h, z), four rows at a time.  The tile's summary rows are loaded and
+// converted once and stay in registers for all of the rows, the next four
+// rows' queries are loaded while the current four are scored, and one barrier
+// per four rows hands the dot products from the lanes that summed them to
+// the wave that owns the row (both buffers alternate).  The dot products and
+// statistics are score_from's and score_stats' in their order, so masks equal
+// per-query selections bit for bit.
+//
+// Bound by vector issue and the LDS reads of the query slices, about equally
+// (680 wave instructions, 256 of them FMAs, and 32 16-byte reads per (row,
+// tile)).  Scoring, merging and deciding in place of one workgroup per
+// (anchor, head, tile) scoring and one per (head, tile) deciding every anchor
+// in turn (64 or 128 workgroups, 137 and 42 us of the time before): 64
+// anchors x 7 rows x 4 heads, 1024 blocks of 64, d 128 170 -> 41 us; 32
+// anchors x 4 rows x 8 heads, 1024 blocks of 32 65 -> 27.7 us.  Measured and
+// dropped: q as scalar operands (an FMA with one runs at half rate: 44.5 us in
+// all) and the statistics of 16 rows a step, four per wave side by side (no
+// faster).
+// (above head_dim 128 the registers of two workgroups per CU: four passes of
+// converted rows; converting them again for each row measured 116 against 25
+// us in all at d 256, 32 anchors x 8 rows x 2 heads)
+template <int D>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 4 : 2)))
+void anchor_rows_kernel(AnchorArgs a) {
+  using S = Dots<D>;
+  constexpr int CH = S::kCh, QW = CH + kQPad, QS = S::kLanes * QW;
+  constexpr int kRows = kWaves;                       // one row per wave's statistics
+  constexpr int kWords = kRows * D / 2;               // query words of kRows rows
+  constexpr int kPer = (kWords + kThreads - 1) / kThreads;
+  __shared__ alignas(16) float q[2][2][kRows * QS];   // [buffer][q, bf16(q^2)]
+  __shared__ alignas(16) float dots[2][2][kRows * kTile];
+  const ScoreArgs& sa = a.score;
+  const int64_t h = blockIdx.y, tile = blockIdx.x, N = sa.n_blocks;
+  const int G = sa.group, r0 = (int)blockIdx.z * a.per;
+  const int r1 = r0 + a.per < a.rows ? r0 + a.per : a.rows;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int c = tid % S::kLanes, sub = tid / S::kLanes;
+
+  // this thread's words of the next kRows rows: row (anchor, g) of each,
+  // advanced by kRows rows at a time (a row past the last one repeats row r0)
+  const int step_a = kRows / G, step_g = kRows % G;
+  int anchor[kPer], g[kPer];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int r = r0 + (tid + k * kThreads) / (D / 2);
+    anchor[k] = r / G;
+    g[k] = r % G;
   }
-  const int lane = threadIdx.x % kWave;
+  uint32_t qw[kPer];
+  auto load = [&](int first) {  // rows first .. first + kRows - 1
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int i = tid + k * kThreads;
+      const bool live = i < kWords && first + i / (D / 2) < r1;
+      const int64_t ga = live ? anchor[k] : r0 / G, gg = live ? g[k] : r0 % G;
+      qw[k] = *reinterpret_cast<const uint32_t*>(sa.query + ga * a.q_as + h * a.q_hs +
+                                                 gg * a.q_gs + 2 * (i % (D / 2)));
+      anchor[k] += step_a;
+      g[k] += step_g;
+      if (g[k] >= G) {
+        g[k] -= G;
+        ++anchor[k];
+      }
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int i = tid + k * kThreads;
+      if (kWords % kThreads != 0 && i >= kWords) continue;
+      const float x0 = bits_f32(qw[k] << 16), x1 = bits_f32(qw[k] & 0xFFFF0000u);
+      const int e = 2 * (i % (D / 2));
+      const int at = i / (D / 2) * QS + (e / CH) * QW + e % CH;
+      q[buf][0][at] = x0;
+      q[buf][0][at + 1] = x1;
+      q[buf][1][at] = round_bf16(x0 * x0);
+      q[buf][1][at + 1] = round_bf16(x1 * x1);
+    }
+  };
+  load(r0);
+  ScoreRaw<D> raw;
+  score_load<D>(sa, h, tile, raw);
+  // the tile's bytes of the mask, which anchor_decide_kernel sets
+  if (blockIdx.z == 0 && tid < kWave && tile * kTile + lane < N)
+    a.mask[h * N + tile * kTile + lane] = 0;
+  stage(0);
+  float km[S::kPasses][CH], el[S::kPasses][CH];
+#pragma unroll
+  for (int ps = 0; ps < S::kPasses; ++ps) {
+    unpack(raw.k[ps], km[ps]);
+    unpack(raw.e[ps], el[ps]);
+  }
+  __syncthreads();
+  int buf = 0;
+  for (int r = r0; r < r1; r += kRows, buf ^= 1) {
+    const bool more = r + kRows < r1;
+    if (more) load(r + kRows);
+#pragma unroll 1
+    for (int j = 0; j < kRows; ++j) {
+      float qv[CH], q2v[CH];
+      lds_read<CH>(&q[buf][0][j * QS + c * QW], qv);
+      lds_read<CH>(&q[buf][1][j * QS + c * QW], q2v);
+#pragma unroll
+      for (int ps = 0; ps < S::kPasses; ++ps) {
+        float s = qv[0] * km[ps][0];
+        float p = q2v[0] * el[ps][0];
+#pragma unroll
+        for (int i = 1; i < CH; ++i) {
+          s = __builtin_fmaf(qv[i], km[ps][i], s);
+          p = __builtin_fmaf(q2v[i], el[ps][i], p);
+        }
+        s = lanes_sum_last<S::kLanes>(s);
+        p = lanes_sum_last<S::kLanes>(p);
+        if (c == S::kLanes - 1) {
+          dots[buf][0][j * kTile + ps * S::kPerPass + sub] = s;
+          dots[buf][1][j * kTile + ps * S::kPerPass + sub] = p;
+        }
+      }
+    }
+    if (more) stage(buf ^ 1);
+    __syncthreads();
+    const int64_t row0 = h * a.rows + r;
+    score_stats(
+        sa, r1 - r < kRows ? r1 - r : kRows, tile, dots[buf][0], dots[buf][1],
+        [&](int j, bool valid, float4 zf) {
+          if (valid) sa.zf[(row0 + j) * sa.z_stride + tile * kTile + lane] = zf;
+        },
+        [&](int j, float4 part) {
+          *reinterpret_cast<float4*>(sa.lse + ((row0 + j) * sa.tile_stride + tile) * 4) = part;
+        });
+  }
+}
+
+// The decisions of anchors [z per, (z + 1) per) of head h for tile `tile`,
+// blockIdx (tile, h, z), one anchor per wave at a time: its rows' risks, the
+// GQA reduction and the fail-safes are decide_finish's, in one wave.  A
+// selected block's byte is set to one (anchor_rows_kernel cleared the tile's
+// bytes; every writer stores the same value, so the order of the workgroups
+// does not matter).
+// kMerged: every row's log Z / log C from lse_merge_kernel; else each wave
+// merges its rows' tile partials itself (at most 64 tiles), in the same order.
+constexpr int kAnchorBatch = 4;  // rows whose statistics are in flight at once
+
+template <bool kMerged>
+__global__ __launch_bounds__(kThreads) void anchor_decide_kernel(AnchorArgs a) {
+  const ScoreArgs& sa = a.score;
+  const int64_t h = blockIdx.y, tile = blockIdx.x, N = sa.n_blocks;
+  const int lane = threadIdx.x % kWave, G = sa.group;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int a0 = (int)blockIdx.z * a.per;
+  const int a1 = a0 + a.per < a.anchors ? a0 + a.per : a.anchors;
   const int64_t b = tile * kTile + lane;
-  if (threadIdx.x < kWave && b < a.n_blocks) mask_out[h * a.n_blocks + b] = (any >> lane) & 1u;
+  const bool valid = b < N;
+  const float vmax = a.max_value_norm[h];
+  const float vnorm = a.value_norm[h * N + (valid ? b : N - 1)];
+  bool any = false;
+  for (int q = a0 + wave; q < a1; q += kWaves) {
+    const int64_t row0 = h * a.rows + (int64_t)q * G;
+    const float4* zf = sa.zf + row0 * sa.z_stride + (valid ? b : N - 1);
+    float acc = 0.0f;
+    bool sel = false, bad = false;
+    for (int g0 = 0; g0 < G; g0 += kAnchorBatch) {
+      float4 f[kAnchorBatch], part[kAnchorBatch];
+      float lz[kAnchorBatch], lc[kAnchorBatch];
+#pragma unroll
+      for (int k = 0; k < kAnchorBatch; ++k) {
+        const int g = g0 + k < G ? g0 + k : G - 1;
+        f[k] = zf[g * sa.z_stride];
+        if constexpr (kMerged) {
+          lz[k] = a.row_lse[(row0 + g) * 2];
+          lc[k] = a.row_lse[(row0 + g) * 2 + 1];
+        } else {
+          part[k] = *reinterpret_cast<const float4*>(
+              sa.lse + ((row0 + g) * sa.tile_stride + (lane < a.n_tiles ? lane : 0)) * 4);
+        }
+      }
+      if constexpr (!kMerged) {
+        // lse_merge_kernel's operations with one tile per lane
+#pragma unroll
+        for (int k = 0; k < kAnchorBatch; ++k) {
+          if (g0 + k >= G) break;
+          const bool in = lane < a.n_tiles;
+          const float sz = inf_to_zero(wave_nanmax_u(in ? part[k].x : kNegInf));
+          const float sc = inf_to_zero(wave_nanmax_u(in ? part[k].z : kNegInf));
+          const float az = in ? part[k].y * exp_hw(part[k].x - sz) : 0.0f;
+          const float ac = in ? part[k].w * exp_hw(part[k].z - sc) : 0.0f;
+          lz[k] = log_hw(wave_sum_u(az)) + sz;
+          lc[k] = log_hw(wave_sum_u(ac)) + sc;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kAnchorBatch; ++k) {
+        if (g0 + k >= G) break;
+        const float r = risk_from(f[k].x, f[k].y, f[k].z, f[k].w, lz[k], lc[k], vmax, vnorm);
+        acc = g0 + k == 0 ? r : acc + r;
+        sel |= a.reduction != kMean && r > a.eps;
+        bad |= !is_finite(r) || !is_finite(lz[k]) || !is_finite(lc[k]);
+      }
+    }
+    if (a.reduction == kMean) sel = acc / (float)G > a.eps;
+    any |= sel || bad;
+  }
+  if (any && valid) a.mask[h * N + b] = 1;
 }
 
 // ---------------------------------------------------------------------------
@@ -2944,7 +3145,7 @@ void step_kernel(StepArgs s) {
   };
   if constexpr (kTiles == 1) {
     score_stats(
-        sa, tile, sh.u.score.sdot, sh.u.score.pdot,
+        sa, G, tile, sh.u.score.sdot, sh.u.score.pdot,
         [&](int g, bool, float4 zf) { sh.zs[g][lane] = zf; },
         [&](int g, float4 part) { publish(tile, g, part); });
     __syncthreads();
@@ -2973,7 +3174,7 @@ void step_kernel(StepArgs s) {
       const bool more = (uint32_t)m + 1u < tset.n;
       if (more) score_load<D>(sa, h, t + W, next);
       score_stats(
-          sa, t, sh.u.score.sdot, sh.u.score.pdot,
+          sa, G, t, sh.u.score.sdot, sh.u.score.pdot,
           [&](int g, bool, float4 zf) {
             sh.tz.z[m][g][lane] = zf.x;
             if (g == wave) tset.zown[m] = zf;
@@ -3206,25 +3407,29 @@ DecideArgs decide_args(const SelectParams& p, const Layout& L) {
   return da;
 }
 
-int launch_score(const SelectParams& p, const Layout& L, int64_t queries = 1) {
+int launch_score(const SelectParams& p, const Layout& L) {
   const ScoreArgs sa = score_args(p, L);
-  const dim3 grid((unsigned)L.n_tiles, (unsigned)(p.heads * queries));
+  const dim3 grid((unsigned)L.n_tiles, (unsigned)p.heads);
   RKV_DISPATCH_DIM(p.dim, D,
                    score_kernel<D><<<grid, dim3(kThreads), score_smem(p.group, p.dim),
                                      p.stream>>>(sa));
   return check_launch("score_kernel");
 }
 
-// With more than 64 tiles per head the rows' log Z / log C are merged once
-// (lse_merge_kernel) and every tile's decision reads them: da.row_lse.
-int launch_lse_merge(const SelectParams& p, const Layout& L, int64_t queries, DecideArgs& da) {
-  if (L.n_tiles <= kWave) return kOk;
-  const int64_t rows = p.heads * queries * p.group;
-  float* row_lse = at<float>(p.ws, L.row_lse);
+// log Z / log C of `rows` rows, merged once per row (lse_merge_kernel).
+int launch_lse_merge(const SelectParams& p, const Layout& L, int64_t rows) {
   lse_merge_kernel<<<dim3((unsigned)((rows + kWaves - 1) / kWaves)), dim3(kThreads), 0,
-                     p.stream>>>(at<float>(p.ws, L.lse), row_lse, rows, L.n_tiles, L.tile_stride);
-  const int rc = check_launch("lse_merge_kernel");
-  if (rc == kOk) da.row_lse = row_lse;
+                     p.stream>>>(at<float>(p.ws, L.lse), at<float>(p.ws, L.row_lse), rows,
+                                 L.n_tiles, L.tile_stride);
+  return check_launch("lse_merge_kernel");
+}
+
+// With more than 64 tiles per head the rows' log Z / log C are merged once
+// and every tile's decision reads them: da.row_lse.
+int lse_for_decisions(const SelectParams& p, const Layout& L, DecideArgs& da) {
+  if (L.n_tiles <= kWave) return kOk;
+  const int rc = launch_lse_merge(p, L, p.heads * p.group);
+  if (rc == kOk) da.row_lse = at<float>(p.ws, L.row_lse);
   return rc;
 }
 
@@ -3235,7 +3440,7 @@ int launch_select(const SelectParams& p, const Layout& L) {
   if (rc) return rc;
   mark(1, p.stream);
   DecideArgs da = decide_args(p, L);
-  if ((rc = launch_lse_merge(p, L, 1, da))) return rc;
+  if ((rc = lse_for_decisions(p, L, da))) return rc;
   decide_kernel<<<dim3((unsigned)L.n_tiles, (unsigned)p.heads), dim3(kThreads), 0, p.stream>>>(
       da, p.accessed);
   rc = check_launch("decide_kernel");
@@ -3243,18 +3448,87 @@ int launch_select(const SelectParams& p, const Layout& L) {
   return rc;
 }
 
-// Batched anchor selection: score every (query, head, tile), then one
-// workgroup per (tile, head) ORs the queries' decisions.  The layout is the
-// one of heads * anchors heads.
-int launch_select_anchors(const SelectParams& p, int64_t anchors) {
+// Batched anchor selection.  The layout is the one of heads * anchors heads
+// (its rows in (head, anchor, group) order); query strides in elements.
+//
+// Rows per workgroup of anchor_rows_kernel: the device holds anchor_slots of
+// its workgroups at once, and a workgroup costs its four-row steps plus about
+// one and a half for the summary rows it waits for; of the ways to cut a
+// head's rows the one whose rounds of workgroups cost least (more, shorter
+// workgroups fill the last round; fewer load the tile's summaries less often).
+template <int D>
+int64_t anchor_slots() {
+  static std::atomic<int> of_dev[64];  // per device; 0 = not asked yet
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 512;
+  int n = of_dev[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    int cus = 0, per_cu = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, anchor_rows_kernel<D>, kThreads,
+                                                     0) != hipSuccess ||
+        cus * per_cu <= 0)
+      return 512;
+    n = cus * per_cu;
+    of_dev[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+constexpr int64_t kAnchorDecides = 2048;  // workgroups anchor_decide_kernel is cut into
+// (row, tile) pairs up to which the decisions merge the rows' log Z / log C
+// themselves: a merge per pair instead of one per row, but one launch less
+// (16384 pairs: 7.1 us in one launch, 4.1 + 3.8 in two; 28672: 9.7 either way).
+constexpr int64_t kAnchorMerges = 20000;
+
+int launch_select_anchors(const SelectParams& p, int64_t anchors, int64_t q_as, int64_t q_hs,
+                          int64_t q_gs) {
   const Layout L = make_layout(p.heads * anchors, p.group, p.dim, p.n_blocks);
-  int rc = launch_score(p, L, anchors);
+  // one dense query: the single selection, two launches
+  if (anchors == 1 && q_hs == p.group * p.dim && q_gs == p.dim) return launch_select(p, L);
+  const int64_t rows = anchors * p.group, cells = L.n_tiles * p.heads;
+  AnchorArgs a;
+  a.score = score_args(p, L);
+  a.row_lse = at<float>(p.ws, L.row_lse);
+  a.value_norm = p.value_norm;
+  a.max_value_norm = p.max_value_norm;
+  a.mask = p.mask;
+  a.q_as = q_as;
+  a.q_hs = q_hs;
+  a.q_gs = q_gs;
+  const int64_t total = p.heads * rows;
+  a.rows = (int)rows;
+  a.anchors = (int)anchors;
+  a.n_tiles = (int)L.n_tiles;
+  a.reduction = p.reduction;
+  a.eps = p.eps;
+  const int64_t steps = (rows + kWaves - 1) / kWaves;
+  int64_t best = steps, best_cost = INT64_MAX, slots = 0;
+  RKV_DISPATCH_DIM(p.dim, D, slots = anchor_slots<D>());
+  for (int64_t cuts = 1; cuts <= steps && cuts <= 64; ++cuts) {
+    const int64_t per = (steps + cuts - 1) / cuts;
+    const int64_t groups = cells * ((steps + per - 1) / per);
+    const int64_t cost = (groups + slots - 1) / slots * (2 * per + 3);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = per;
+    }
+  }
+  a.per = (int)(best * kWaves);
+  const dim3 grid((unsigned)L.n_tiles, (unsigned)p.heads,
+                  (unsigned)((rows + a.per - 1) / a.per));
+  RKV_DISPATCH_DIM(p.dim, D, anchor_rows_kernel<D><<<grid, dim3(kThreads), 0, p.stream>>>(a));
+  int rc = check_launch("anchor_rows_kernel");
   if (rc) return rc;
-  DecideArgs da = decide_args(p, L);
-  da.write_mask = false;  // the mask only stands in for the (absent) anchor input
-  if ((rc = launch_lse_merge(p, L, anchors, da))) return rc;
-  anchor_decide_kernel<<<dim3((unsigned)L.n_tiles, (unsigned)p.heads), dim3(kThreads), 0,
-                         p.stream>>>(da, (int)anchors, (int)p.heads, p.mask);
+  const bool merged = L.n_tiles > kWave || total * L.n_tiles > kAnchorMerges;
+  if (merged && (rc = launch_lse_merge(p, L, total))) return rc;
+  // (at least one anchor per wave)
+  const int64_t cuts = std::min((anchors + kWaves - 1) / kWaves,
+                                std::max<int64_t>(kAnchorDecides / cells, 1));
+  a.per = (int)((anchors + cuts - 1) / cuts);
+  const dim3 decide((unsigned)L.n_tiles, (unsigned)p.heads,
+                    (unsigned)((anchors + a.per - 1) / a.per));
+  if (merged) anchor_decide_kernel<true><<<decide, dim3(kThreads), 0, p.stream>>>(a);
+  else anchor_decide_kernel<false><<<decide, dim3(kThreads), 0, p.stream>>>(a);
   return check_launch("anchor_decide_kernel");
 }
 
@@ -3517,7 +3791,7 @@ int launch_decode(const SelectParams& p, const Layout& L, const DecodeBuffers& b
   int rc = launch_score(p, L);
   if (rc) return rc;
   mark(1, p.stream);
-  if ((rc = launch_lse_merge(p, L, 1, aa.decide))) return rc;
+  if ((rc = lse_for_decisions(p, L, aa.decide))) return rc;
   rc = kUnsupported;
   RKV_DISPATCH_DIM(p.dim, D, rc = launch_attend<D>(aa, rows, tiles, p.stream));
   if (rc) return rc;
@@ -3724,6 +3998,33 @@ extern "C" int rkv_select(const void* query, const void* key_mean, const void* e
   return launch_select(p, L);
 }
 
+extern "C" int rkv_select_anchors_strided(
+    const void* queries, int64_t q_anchor_stride, int64_t q_head_stride, int64_t q_row_stride,
+    const void* key_mean, const void* ellipsoid, const float* value_norm,
+    const float* max_value_norm, int64_t heads, int64_t group, int64_t dim, int64_t n_blocks,
+    int64_t block_size, int64_t prompt_length, float eps, int reduction, int64_t anchors,
+    uint8_t* mask_out, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  clear_error();
+  const char* who = "rkv_select_anchors";
+  if (anchors <= 0 || anchors > 65535)
+    return set_error(kInvalidArgument, "%s: anchors must be in 1..65535", who);
+  if (heads > 0 && heads * anchors > 65535)
+    return set_error(kUnsupported, "%s: heads x anchors exceeds 65535", who);
+  if (q_anchor_stride % 8 || q_head_stride % 8 || q_row_stride % 8)
+    return set_error(kInvalidArgument, "%s: query strides must be multiples of 8 elements", who);
+  SelectParams p{queries, key_mean, ellipsoid, value_norm, max_value_norm, heads, group, dim,
+                 n_blocks, block_size, prompt_length, eps, reduction, nullptr, mask_out,
+                 nullptr, nullptr, nullptr, workspace, workspace_bytes, stream};
+  Layout L;
+  int rc = validate_select(p, who, L);
+  if (rc) return rc;
+  const Layout LA = make_layout(heads * anchors, group, dim, n_blocks);
+  if (workspace_bytes < (size_t)LA.total)
+    return set_error(kWorkspaceTooSmall, "%s: workspace needs %lld bytes (rkv_workspace_bytes of "
+                     "heads x anchors heads)", who, (long long)LA.total);
+  return launch_select_anchors(p, anchors, q_anchor_stride, q_head_stride, q_row_stride);
+}
+
 extern "C" int rkv_select_anchors(const void* queries, const void* key_mean,
                                   const void* ellipsoid, const float* value_norm,
                                   const float* max_value_norm, int64_t heads, int64_t group,
@@ -3731,23 +4032,10 @@ extern "C" int rkv_select_anchors(const void* queries, const void* key_mean,
                                   int64_t prompt_length, float eps, int reduction,
                                   int64_t anchors, uint8_t* mask_out, void* workspace,
                                   size_t workspace_bytes, hipStream_t stream) {
-  clear_error();
-  if (anchors <= 0 || anchors > 65535)
-    return set_error(kInvalidArgument, "rkv_select_anchors: anchors must be in 1..65535");
-  if (heads > 0 && heads * anchors > 65535)
-    return set_error(kUnsupported, "rkv_select_anchors: heads x anchors exceeds 65535");
-  SelectParams p{queries, key_mean, ellipsoid, value_norm, max_value_norm, heads, group, dim,
-                 n_blocks, block_size, prompt_length, eps, reduction, nullptr, mask_out,
-                 nullptr, nullptr, nullptr, workspace, workspace_bytes, stream};
-  Layout L;
-  int rc = validate_select(p, "rkv_select_anchors", L);
-  if (rc) return rc;
-  const Layout LA = make_layout(heads * anchors, group, dim, n_blocks);
-  if (workspace_bytes < (size_t)LA.total)
-    return set_error(kWorkspaceTooSmall,
-                     "rkv_select_anchors: workspace needs %lld bytes (rkv_workspace_bytes of "
-                     "heads x anchors heads)", (long long)LA.total);
-  return launch_select_anchors(p, anchors);
+  return rkv_select_anchors_strided(queries, heads * group * dim, group * dim, dim, key_mean,
+                                    ellipsoid, value_norm, max_value_norm, heads, group, dim,
+                                    n_blocks, block_size, prompt_length, eps, reduction, anchors,
+                                    mask_out, workspace, workspace_bytes, stream);
 }
 
 extern "C" int rkv_decode(const void* query, const void* key_mean, const void* ellipsoid,

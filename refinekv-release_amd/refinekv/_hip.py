@@ -66,6 +66,9 @@ def _bind(lib):
     lib.rkv_select_anchors.argtypes = [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64,
                                        _f32, _int, _i64, _p, _p, _size, _p]
     lib.rkv_select_anchors.restype = _int
+    lib.rkv_select_anchors_strided.argtypes = ([_p, _i64, _i64, _i64]
+                                               + lib.rkv_select_anchors.argtypes[1:])
+    lib.rkv_select_anchors_strided.restype = _int
     lib.rkv_decode.argtypes = [_p, _p, _p, _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _i64, _p,
                                _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64, _i64, _i64, _f32,
                                _int, _p, _p, _p, _p, _p, _size, _p]
@@ -269,12 +272,13 @@ def select(query, summary, config, workspace=None, risk_out=None, stats_out=None
 
 
 def select_anchors(queries, summary, config, workspace=None):
-    """Union of the expanded-block masks of queries (H, G, A, D): one launch
-    scores every (query, head, tile), one ORs the decisions.  The scratch is
-    its own workspace entry (sized for H * A heads), apart from the decode
-    step's."""
+    """Union of the expanded-block masks of queries (H, G, A, D): every query
+    row is scored in one launch, then the rows' statistics are merged and
+    the decisions ORed.  The scratch is its own workspace entry (sized for
+    H * A heads), apart from the decode step's."""
     heads, group, count, dim = queries.shape
-    q = queries.permute(2, 0, 1, 3).contiguous()  # (A, H, G, D)
+    aligned = queries.is_contiguous() and queries.data_ptr() % 16 == 0
+    q = queries if aligned else _row_aligned(queries, 16)
     n_blocks = summary.num_blocks
     shape = (heads * count, group, dim, n_blocks)
     nbytes = workspace_bytes(*shape)
@@ -284,10 +288,11 @@ def select_anchors(queries, summary, config, workspace=None):
         if workspace is not None:
             workspace["hip_anchor_scratch"] = scratch
     mask = torch.empty(heads, n_blocks, device=queries.device, dtype=torch.bool)
-    rc = lib().rkv_select_anchors(
-        _ptr(q), *_summary_args(summary), heads, group, dim, n_blocks, summary.block_size,
-        summary.prompt_length, float(config.eps), REDUCTION_CODES[config.gqa_reduction], count,
-        _ptr(mask), _ptr(scratch), scratch.numel(), _stream(queries.device))
+    rc = lib().rkv_select_anchors_strided(
+        _ptr(q), q.stride(2), q.stride(0), q.stride(1), *_summary_args(summary), heads, group,
+        dim, n_blocks, summary.block_size, summary.prompt_length, float(config.eps),
+        REDUCTION_CODES[config.gqa_reduction], count, _ptr(mask), _ptr(scratch), scratch.numel(),
+        _stream(queries.device))
     _check(rc, "rkv_select_anchors")
     return mask
 
