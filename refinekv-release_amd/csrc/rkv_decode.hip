@@ -1896,32 +1896,50 @@ struct LaneCombine {
 };
 
 // The matrix-core path's LDS: each wave's staged value chunks, then each
-// wave's state for the combine.
-template <int D, int GBM>
+// wave's state for the combine.  kOver: the state takes the place of the
+// wave's own chunks, once its ring has ended (its last wait leaves no load in
+// flight), for the attend kernel, whose z rows take the space without a
+// workgroup per CU lost; the step keeps them apart (0.6 % faster at 131072
+// tokens).
+template <int D, int GBM, bool kOver>
 struct MmaCombine {
   MmaStage<D> stage[kWaves];
   MmaOut<D, GBM> mma[kWaves];
+  __device__ __forceinline__ MmaOut<D, GBM>& out(int w) { return mma[w]; }
+  __device__ __forceinline__ const MmaOut<D, GBM>& out(int w) const { return mma[w]; }
+  __device__ __forceinline__ MmaStage<D>& chunks(int w) { return stage[w]; }
+};
+template <int D, int GBM>
+struct MmaCombine<D, GBM, true> {
+  union Wave {
+    MmaStage<D> stage;
+    MmaOut<D, GBM> out;
+  };
+  Wave of[kWaves];
+  __device__ __forceinline__ MmaOut<D, GBM>& out(int w) { return of[w].out; }
+  __device__ __forceinline__ const MmaOut<D, GBM>& out(int w) const { return of[w].out; }
+  __device__ __forceinline__ MmaStage<D>& chunks(int w) { return of[w].stage; }
 };
 
 // The four waves' published states -> one (m, l, acc) per query row j < gn,
 // in a fixed order: put(j, d, (acc[d], acc[d + 1]), m, l) for each column
 // pair d of each row (after a barrier that follows every wave's publish).
-template <int D, int GBM, typename Put>
-__device__ __forceinline__ void mma_combine(const MmaCombine<D, GBM>& cmb, int gn, Put put) {
+template <int D, int GBM, bool kOver, typename Put>
+__device__ __forceinline__ void mma_combine(const MmaCombine<D, GBM, kOver>& cmb, int gn, Put put) {
   for (int idx = 2 * (int)threadIdx.x; idx < gn * D; idx += 2 * kThreads) {
     const int j = idx / D, d = idx % D;
     float M = kNegInf;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) M = fmaxf(M, cmb.mma[w].ml[j][0]);
+    for (int w = 0; w < kWaves; ++w) M = fmaxf(M, cmb.out(w).ml[j][0]);
     float a0 = 0.0f, a1 = 0.0f, l = 0.0f;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
-      const float mw = cmb.mma[w].ml[j][0];
+      const float mw = cmb.out(w).ml[j][0];
       const float e = mw == kNegInf ? 0.0f : __builtin_amdgcn_exp2f((mw - M) * kLog2e);
-      const float2 av = *reinterpret_cast<const float2*>(&cmb.mma[w].acc[j][d]);
+      const float2 av = *reinterpret_cast<const float2*>(&cmb.out(w).acc[j][d]);
       a0 = __builtin_fmaf(av.x, e, a0);
       a1 = __builtin_fmaf(av.y, e, a1);
-      l = __builtin_fmaf(cmb.mma[w].ml[j][1], e, l);
+      l = __builtin_fmaf(cmb.out(w).ml[j][1], e, l);
     }
     put(j, d, make_float2(a0, a1), M, l);
   }
@@ -2499,9 +2517,10 @@ __device__ __forceinline__ void mma_stage_reps(const AttendArgs& a, int64_t h, u
 // the partials.
 template <int D, int GBM, bool kFused, int kTiles = 1>
 __device__ __forceinline__ void attend_tile_mma(const AttendArgs& a, DecideShared& dsh,
-                                                MmaCombine<D, GBM>& cmb, const StepCtx* sx,
+                                                MmaCombine<D, GBM, !kFused>& cmb, const StepCtx* sx,
                                                 const MmaLoads<D>& ld, int64_t h, uint32_t wk,
-                                                const TileSet<kTiles, GBM>* tset = nullptr) {
+                                                const TileSet<kTiles, GBM>* tset = nullptr,
+                                                float (*zsh)[kTile] = nullptr) {
   constexpr bool kMulti = kTiles > 1;
   static_assert(!kMulti || (kFused && GBM == 4), "several tiles: one-launch step, 4-row passes");
   using S = MmaShape<D>;
@@ -2523,7 +2542,7 @@ __device__ __forceinline__ void attend_tile_mma(const AttendArgs& a, DecideShare
   const uint32_t copies = kMulti ? 1u : (W - tile + T - 1u) / T;
   const uint32_t copy = kMulti ? 0u : wk / T;
 
-  MmaStage<D>& stage = cmb.stage[wave];
+  MmaStage<D>& stage = cmb.chunks(wave);
   unsigned long long* stamps = nullptr;  // (phase stamps build)
   if constexpr (kFused) stamps = sx->stats.stamps;
   (void)stamps;
@@ -2695,7 +2714,7 @@ __device__ __forceinline__ void attend_tile_mma(const AttendArgs& a, DecideShare
   if constexpr (kMulti) {
     decide_tiles<kTiles, GBM>(da, h, wk, W, *tset, dsh, sx->stats, bits, count);
   } else {
-    bits[0] = decide_finish<kFused, false, GBM>(da, h, tile, ld.din, dsh, nullptr, plist, count,
+    bits[0] = decide_finish<kFused, false, GBM>(da, h, tile, ld.din, dsh, zsh, plist, count,
                                            kFused ? &sx->stats : nullptr);
   }
   RKV_STAMP(stamps, kStDecided, tid == 0);
@@ -2712,6 +2731,20 @@ __device__ __forceinline__ void attend_tile_mma(const AttendArgs& a, DecideShare
     for (int m = 0; m < kTiles; ++m) blocks += (uint32_t)__popcll(bits[m]);
     set_rows(blocks);
     if (spec) pre_issue();
+  }
+
+  // Three kernels: the logits of the wave's representative chunk from the z
+  // rows that the decision left in LDS, read before the ring's loads are
+  // issued (an LDS read behind them would wait for them).  Loaded from the
+  // score kernel's rows again they were a round trip through L2 in the chain
+  // between the decision and the first fold of each of a head's 512 tiles
+  // (8 heads x 524288 tokens at block 16: 95.2 us a layer, now 91.0).
+  float rep_z[4] = {};
+  if constexpr (!kFused) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      rep_z[i] = zsh[g0 + ((lane & 15) < gn ? lane & 15 : 0)]
+                    [16u * wave + 4u * (uint32_t)(lane >> 4) + i];
   }
 
   // ---- the ring -------------------------------------------------------------
@@ -2731,7 +2764,7 @@ __device__ __forceinline__ void attend_tile_mma(const AttendArgs& a, DecideShare
       float z;
       if constexpr (kMulti) z = tset->z[j < kTiles ? j : 0][gg][tb];
       else if constexpr (kFused) z = sx->stats.zs[gg][tb].x;
-      else z = da.zf[(h * G + g0 + gg) * da.z_stride + (b < N ? b : N - 1)].x;
+      else z = rep_z[i];
       x[i] = live ? z : kNegInf;
     }
   };
@@ -2838,7 +2871,7 @@ __device__ __forceinline__ void attend_tile_mma(const AttendArgs& a, DecideShare
 
   // ---- the four waves -> one partial per query row, through LDS ------------
   RKV_STAMP(stamps, kStPagesWave0, tid == 0);
-  mma_publish<D, GBM>(st, cmb.mma[wave]);
+  mma_publish<D, GBM>(st, cmb.out(wave));
   __syncthreads();
   RKV_STAMP(stamps, kStCombine, tid == 0);
   uint32_t tag = 0u;
@@ -2847,7 +2880,7 @@ __device__ __forceinline__ void attend_tile_mma(const AttendArgs& a, DecideShare
     tag = __builtin_amdgcn_readfirstlane(*sx->stats.tag);
     nan_partial = *sx->stats.gave_up != 0u;
   }
-  mma_combine<D, GBM>(cmb, gn, [&](int j, int d, float2 acc, float M, float l) {
+  mma_combine(cmb, gn, [&](int j, int d, float2 acc, float M, float l) {
     if (nan_partial) l = bits_f32(0x7FC00000u);
     const int64_t at = (h * G + g0 + j) * da.tile_stride + wk;
     if constexpr (kFused) {
@@ -2887,11 +2920,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void attend_kernel(AttendArgs a) {
   __shared__ alignas(16) DecideShared dsh;
   if constexpr (D <= kMmaMaxDim) {
-    __shared__ alignas(16) MmaCombine<D, GBM> cmb;
+    __shared__ alignas(16) MmaCombine<D, GBM, true> cmb;
     const int64_t h = blockIdx.y;
     const uint32_t wk = blockIdx.x;
     const MmaLoads<D> ld = mma_issue<D, GBM, false>(a, h, wk);
-    attend_tile_mma<D, GBM, false>(a, dsh, cmb, nullptr, ld, h, wk);
+    __shared__ float zsh[kMaxGroup][kTile];  // z of the tile, from the decision's loads
+    attend_tile_mma<D, GBM, false>(a, dsh, cmb, nullptr, ld, h, wk,
+                                   static_cast<const TileSet<1, GBM>*>(nullptr), zsh);
   } else {
     __shared__ alignas(16) LaneCombine<D, GBM> cmb;
     const AttendLoads<D, GBM> ld = attend_issue<D, GBM>(a, blockIdx.y, blockIdx.x);
@@ -2932,7 +2967,7 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 && GBM <= 8 ? 2 : 1)))
 void dense_kernel(DenseArgs a) {
   using S = MmaShape<D>;
   constexpr uint32_t kRowBytes = D * 2;
-  __shared__ alignas(16) MmaCombine<D, GBM> cmb;
+  __shared__ alignas(16) MmaCombine<D, GBM, false> cmb;
   const int64_t h = blockIdx.y;
   const uint32_t sp = blockIdx.x, splits = (uint32_t)a.splits;
   const int G = a.group, g0 = blockIdx.z * GBM, gn = min(GBM, G - g0);
@@ -2954,7 +2989,7 @@ void dense_kernel(DenseArgs a) {
   const auto vres = buffer_view(a.values + h * a.v_hs, a.cap ? (a.cap - 1u) * vts + kRowBytes : 0u);
   Bf16x8 qop[S::kSteps];
   mma_query<D, GBM>(qop, a.query + h * (int64_t)G * D, g0, G);
-  MmaStage<D>& stage = cmb.stage[wave];
+  MmaStage<D>& stage = cmb.chunks(wave);
   MmaState<D> st;
   st.m = kNegInf;
   st.lsum = 0.0f;
@@ -2982,9 +3017,9 @@ void dense_kernel(DenseArgs a) {
         }
         mma_fold<D>(st, x, stage.bytes[sidx]);
       });
-  mma_publish<D, GBM>(st, cmb.mma[wave]);
+  mma_publish<D, GBM>(st, cmb.out(wave));
   __syncthreads();
-  mma_combine<D, GBM>(cmb, gn, [&](int j, int d, float2 acc, float M, float l) {
+  mma_combine(cmb, gn, [&](int j, int d, float2 acc, float M, float l) {
     const int64_t at = (h * G + g0 + j) * (int64_t)splits + sp;
     *reinterpret_cast<float2*>(a.part_acc + at * D + d) = acc;
     if (d == 0) a.part_ml[at] = make_float2(M, l);
@@ -3040,7 +3075,7 @@ struct StepShared {
       alignas(16) float pdot[GBM * kTile];
       alignas(16) float q[score_q_floats_max(GBM, D)];
     } score;
-    alignas(16) MmaCombine<D, GBM> cmb;
+    alignas(16) MmaCombine<D, GBM, false> cmb;
   } u;
 #if defined(RKV_PHASE_STAMPS)
   unsigned long long stamps[kStamps];
