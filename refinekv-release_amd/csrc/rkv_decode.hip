@@ -3266,7 +3266,7 @@ struct MergeArgs {
 // and the stripes combine by lane exchanges and one LDS step; folded one
 // partial after another (16 per lane, then 32 stripes in one lane, then the
 // access count) the 512 partials of 32 rows at head_dim 128 took 9.1 us,
-// now 4.8, and the dense decode's 64 splits 4.9, now 4.0.
+// now 4.5, and the dense decode's 64 splits 4.9, now 4.0.
 constexpr int kMergeFewParts = 128;
 
 template <int kMergeD, int kMergeBatch>
