@@ -3261,20 +3261,49 @@ struct MergeArgs {
 // (the dense decode's splits, a head of up to 128 tiles): 32 columns, 8
 // stripes of batches of 8; many (more tiles): 8 columns, so that the
 // workgroups fill the device and each stripe takes one or two batches of 16.
-// Latency bounds it: one round trip for a batch, then the fold.  A batch's
-// maximum is taken first, so its exponentials do not wait for one another,
-// and the stripes combine by lane exchanges and one LDS step; folded one
-// partial after another (16 per lane, then 32 stripes in one lane, then the
-// access count) the 512 partials of 32 rows at head_dim 128 took 9.1 us,
-// now 4.5, and the dense decode's 64 splits 4.9, now 4.0.
+// A stripe folds its partials one after another, as an online softmax, then
+// one lane per column folds the stripes in order: this order is part of the
+// result (bf16 outputs change where fp32 sums are taken in another).
+// Latency bounds it: one round trip for a batch, then the fold.  The weights
+// of a batch are taken before its sums (merge_fold), so its exponentials do
+// not wait for one another, and the access count has a workgroup of its own.
 constexpr int kMergeFewParts = 128;
+
+// Merges N partials (m, l, acc), in order, into (mx, num, den): the running
+// sums are rescaled where a partial's m is above the maximum so far, else the
+// partial is; one that is empty (l not above 0) is skipped.  The maxima before
+// each partial, and so the weights, do not depend on the sums: only a multiply
+// and an add per partial are in the chain.  (A skipped partial adds -0, which
+// leaves any sum as it is.)
+template <int N>
+__device__ __forceinline__ void merge_fold(const float (&m)[N], const float (&l)[N],
+                                           const float (&acc)[N], float& mx, float& num,
+                                           float& den) {
+  float w[N], lv[N], av[N];
+  bool up[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const bool live = l[u] > 0.0f;
+    const float d = live ? m[u] - mx : 0.0f;
+    lv[u] = live ? l[u] : -0.0f;
+    av[u] = live ? acc[u] : -0.0f;
+    up[u] = d > 0.0f;
+    w[u] = __builtin_amdgcn_exp2f(-fabsf(d) * kLog2e);
+    mx = up[u] ? m[u] : mx;
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    num = up[u] ? num * w[u] + av[u] : __builtin_fmaf(av[u], w[u], num);
+    den = up[u] ? den * w[u] + lv[u] : __builtin_fmaf(lv[u], w[u], den);
+  }
+}
 
 template <int kMergeD, int kMergeBatch>
 __global__ __launch_bounds__(kThreads) void merge_kernel(MergeArgs a) {
   constexpr int kMergeK = kThreads / kMergeD;  // partial stripes
-  __shared__ float sm[kWaves], sd[kWaves], sn[kWaves][kMergeD];
+  __shared__ float sm[kMergeK], sn[kMergeK][kMergeD + 1];  // the columns' sums, then den
   __shared__ unsigned long long wsum[kWaves];
-  const int tid = threadIdx.x, wave = tid / kWave;
+  const int tid = threadIdx.x;
   // the step's access count: sum of the tile counts, added once, by a
   // workgroup of its own beside the rows'
   if (blockIdx.x == (unsigned)a.rows) {
@@ -3294,7 +3323,7 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(MergeArgs a) {
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, kWave);
-    if (tid % kWave == 0) wsum[wave] = s;
+    if (tid % kWave == 0) wsum[tid / kWave] = s;
     __syncthreads();
     if (tid == 0) atomicAdd(a.accessed, ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3]);
     return;
@@ -3319,61 +3348,39 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(MergeArgs a) {
       av[u] = pa[(int64_t)ii * D];
       if (i >= P) lv[u] = 0.0f;
     }
-    // the batch's maximum first, so that its weights do not wait for one
-    // another; an empty partial (l not above 0) weighs nothing
-    float top = mx;
-#pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u) {
-      const bool live = lv[u] > 0.0f;
-      mv[u] = live ? mv[u] : kNegInf;
-      lv[u] = live ? lv[u] : 0.0f;
-      av[u] = live ? av[u] : 0.0f;
-      top = fmaxf(top, mv[u]);
-    }
-    const float ms = top == kNegInf ? 0.0f : top;
-    const float keep = __builtin_amdgcn_exp2f((mx - ms) * kLog2e);
-    num *= keep;
-    den *= keep;
-    mx = top;
-#pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u) {
-      const float e = __builtin_amdgcn_exp2f((mv[u] - ms) * kLog2e);
-      num = __builtin_fmaf(av[u], e, num);
-      den = __builtin_fmaf(lv[u], e, den);
-    }
+    merge_fold(mv, lv, av, mx, num, den);
   }
-  // the stripes of a wave (lanes with the same column), then the four waves
-  float top = mx;
-#pragma unroll
-  for (int o = kMergeD; o < kWave; o <<= 1) top = fmaxf(top, __shfl_xor(top, o, kWave));
-  {
-    const float e = __builtin_amdgcn_exp2f((mx - (top == kNegInf ? 0.0f : top)) * kLog2e);
-    num *= e;
-    den *= e;
-  }
-#pragma unroll
-  for (int o = kMergeD; o < kWave; o <<= 1) {
-    num += __shfl_xor(num, o, kWave);
-    den += __shfl_xor(den, o, kWave);
-  }
-  if (tid % kWave < kMergeD) sn[wave][dl] = num;
-  if (tid % kWave == 0) {
-    sm[wave] = top;
-    sd[wave] = den;
+  sn[kk][dl] = num;
+  if (dl == 0) {
+    sm[kk] = mx;
+    sn[kk][kMergeD] = den;
   }
   __syncthreads();
-  if (tid < kMergeD && d < D) {
-    const float m2 = fmaxf(fmaxf(sm[0], sm[1]), fmaxf(sm[2], sm[3]));
-    const float ms = m2 == kNegInf ? 0.0f : m2;
-    float n2 = 0.0f, d2 = 0.0f;
+  if (tid >= kWave) return;
+  // the stripes in order, as merge_fold: lane j takes stripe j's weight, then
+  // each lane folds a column (lane kMergeD the denominators)
+  float x[kMergeK];
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-      const float e = __builtin_amdgcn_exp2f((sm[w] - ms) * kLog2e);
-      n2 = __builtin_fmaf(sn[w][tid], e, n2);
-      d2 = __builtin_fmaf(sd[w], e, d2);
-    }
-    a.out[r * D + d] = bf16_rne(n2 / fmaxf(d2, 1e-30f));
+  for (int j = 0; j < kMergeK; ++j) x[j] = sn[j][tid < kMergeD ? tid : kMergeD];
+  const int js = tid < kMergeK ? tid : kMergeK - 1;
+  const bool live = tid < kMergeK && sn[js][kMergeD] > 0.0f;
+  float top = live ? sm[js] : kNegInf;
+  const float mine = top;
+#pragma unroll
+  for (int o = 1; o < kMergeK; o <<= 1) top = fmaxf(top, __shfl_up(top, o, kWave));
+  const float prev = __shfl_up(top, 1, kWave);
+  const float d0 = mine - (tid ? prev : kNegInf);
+  const uint64_t lives = __ballot(live), ups = __ballot(live && d0 > 0.0f);
+  const float w = __builtin_amdgcn_exp2f(-fabsf(d0) * kLog2e);
+  float sum = 0.0f;
+#pragma unroll
+  for (int j = 0; j < kMergeK; ++j) {
+    if (!((lives >> j) & 1u)) continue;
+    const float wj = readlane(w, j);
+    sum = (ups >> j) & 1u ? sum * wj + x[j] : __builtin_fmaf(x[j], wj, sum);
   }
+  const float total = readlane(sum, kMergeD);
+  if (tid < kMergeD && d < D) a.out[r * D + d] = bf16_rne(sum / fmaxf(total, 1e-30f));
 }
 
 // ---------------------------------------------------------------------------
