@@ -69,7 +69,8 @@ __device__ __forceinline__ void cols_f32(const RawCols<In, N>& r, float (&x)[N])
 }
 
 // Buffer view of one block's rows: a scalar base and 32-bit byte offsets.
-// Reads at or past `bytes` return 0 and writes there are dropped.
+// Reads whose lane offset is at or past `bytes` return 0 and writes there are
+// dropped (a scalar offset is not part of that check).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_view(const void* base, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, bytes, 0x00020000);
 }
@@ -94,20 +95,23 @@ __device__ __forceinline__ RawCols<In, N> buf_cols(__amdgpu_buffer_rsrc_t r, int
   return c;
 }
 
+// The whole offset is the lane's: a view's bounds check does not cover the
+// scalar offset, and stores past the end (rows past the prompt in the cache,
+// any row of a tensor that is not written) have to be dropped.
 template <class In, int N>
-__device__ __forceinline__ void buf_store_cols(__amdgpu_buffer_rsrc_t r, int voff, int soff,
+__device__ __forceinline__ void buf_store_cols(__amdgpu_buffer_rsrc_t r, int voff,
                                                const RawCols<In, N>& c) {
   constexpr int W = RawCols<In, N>::W;
   typedef unsigned int U2 __attribute__((ext_vector_type(2)));
   typedef unsigned int U4 __attribute__((ext_vector_type(4)));
   if constexpr (W == 1) {
-    __builtin_amdgcn_raw_buffer_store_b32(c.w[0], r, voff, soff, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(c.w[0], r, voff, 0, 0);
   } else if constexpr (W == 2) {
     const U2 v = {c.w[0], c.w[1]};
-    __builtin_amdgcn_raw_buffer_store_b64(v, r, voff, soff, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(v, r, voff, 0, 0);
   } else {
     const U4 v = {c.w[0], c.w[1], c.w[2], c.w[3]};
-    __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, soff, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, 0, 0);
   }
 }
 
@@ -360,8 +364,8 @@ __device__ __forceinline__ void summary_passes(
 #pragma unroll
       for (int i = 0; i < kStore; ++i) {
         if (on1 && dst[i].narrow) {
-          buf_store_cols<In, CPL>(dst[i].k, col * E, t * dst[i].ks, rk);
-          buf_store_cols<In, CPL>(dst[i].v, col * E, t * dst[i].vs, rv);
+          buf_store_cols<In, CPL>(dst[i].k, col * E + t * dst[i].ks, rk);
+          buf_store_cols<In, CPL>(dst[i].v, col * E + t * dst[i].vs, rv);
         }
       }
     }

@@ -296,3 +296,21 @@ def test_transposed_reads_are_waited_for_before_use(kernels):
             assert not _unwaited_transposed_reads(block.splitlines()[1:]), m.group(1)
             checked += block.count("ds_read_b64_tr_b16")
     assert checked > 0
+
+
+@needs_tools
+def test_summary_stores_carry_their_whole_offset_per_lane(kernels):
+    """A buffer store's bounds check covers the lane's offset, not the scalar
+    one: the summary's stores past a view's end (rows past the prompt in the
+    cache, the rows of a tensor that is not written) are dropped only where
+    the scalar offset is 0."""
+    stores = 0
+    for obj in {res["obj"] for name, res in kernels.items() if "summary" in name}:
+        text = subprocess.run([os.path.join(LLVM, "llvm-objdump"), "-d", obj], check=True,
+                              capture_output=True, text=True).stdout
+        for line in text.splitlines():
+            m = re.search(r"\bbuffer_store_\w+ \S+, \S+, s\[[\d:]+\], (\S+)", line)
+            if m:
+                stores += 1
+                assert m.group(1) == "0", line
+    assert stores

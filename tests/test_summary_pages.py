@@ -26,6 +26,11 @@ CASES = [
     (torch.float32, 256, 64, 64 * 2 + 1),
     (torch.bfloat16, 32, 16, 5),
     (torch.bfloat16, 128, 32, 32 * 6),
+    # whole blocks that go out through registers: with dense keys and strided
+    # values only the values' pages are written
+    (torch.float32, 128, 32, 32 * 3),
+    (torch.float32, 256, 64, 64 * 2),
+    (torch.bfloat16, 256, 16, 16 * 9),
 ]
 
 
