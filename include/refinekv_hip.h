@@ -166,7 +166,7 @@ int rkv_select_anchors(const void* queries, const void* key_mean, const void* el
 /* rkv_select_anchors for queries in any order of axes: query row (anchor,
  * head, g) starts q_anchor_stride, q_head_stride and q_row_stride elements
  * (multiples of 8) apart, dim dense, e.g. the (heads, group, anchors, dim)
- * rows of a projection. */
+ * rows of a projection.  The stride of an axis of length one is not read. */
 int rkv_select_anchors_strided(const void* queries, int64_t q_anchor_stride,
                                int64_t q_head_stride, int64_t q_row_stride, const void* key_mean,
                                const void* ellipsoid, const float* value_norm,

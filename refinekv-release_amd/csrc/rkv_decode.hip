@@ -4091,6 +4091,10 @@ extern "C" int rkv_select_anchors_strided(
     return set_error(kInvalidArgument, "%s: anchors must be in 1..65535", who);
   if (heads > 0 && heads * anchors > 65535)
     return set_error(kUnsupported, "%s: heads x anchors exceeds 65535", who);
+  // (an axis of length one has no stride: a tensor may carry any value there)
+  if (anchors == 1) q_anchor_stride = heads * group * dim;
+  if (heads == 1) q_head_stride = group * dim;
+  if (group == 1) q_row_stride = dim;
   if (q_anchor_stride % 8 || q_head_stride % 8 || q_row_stride % 8)
     return set_error(kInvalidArgument, "%s: query strides must be multiples of 8 elements", who);
   SelectParams p{queries, key_mean, ellipsoid, value_norm, max_value_norm, heads, group, dim,

@@ -60,6 +60,25 @@ def test_union_equals_select_per_anchor(heads, group, dim, block, prompt, anchor
             assert torch.equal(got, want), (name, eps)
 
 
+@pytest.mark.parametrize("heads,group,anchors", [(8, 4, 1), (4, 1, 20), (1, 3, 5), (1, 1, 1)])
+def test_axes_of_length_one_may_have_any_stride(heads, group, anchors):
+    """The stride of a length-one axis says nothing: is_contiguous() ignores
+    it, and views carry odd values there."""
+    keys, values, queries = inputs(heads, group, 64, 32, 1000, anchors)
+    cfg = RefineKVConfig(backend="hip", eps=0.05)
+    summary = build_summary(keys, values, cfg)
+    shape = queries.shape
+    strides = [1 if n == 1 else s for n, s in zip(shape, queries.stride())]
+    view = queries.as_strided(shape, strides)
+    assert view.is_contiguous() and torch.equal(view, queries)
+    assert torch.equal(select_blocks_union(view, summary, cfg, workspace={}),
+                       union(queries, summary, cfg))
+    # a column of a wider tensor
+    wide = torch.cat([queries, queries[..., :1]], -1)[..., :64]
+    assert torch.equal(select_blocks_union(wide, summary, cfg, workspace={}),
+                       union(queries, summary, cfg))
+
+
 @pytest.mark.parametrize("reduction", ["any", "max", "mean"])
 @pytest.mark.parametrize("what", ["inf query", "nan query", "zero query", "nan block", "huge"])
 def test_union_with_values_that_are_not_finite(what, reduction):
