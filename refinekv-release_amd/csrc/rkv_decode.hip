@@ -3243,7 +3243,7 @@ void step_kernel(StepArgs s) {
 
 // ---------------------------------------------------------------------------
 // Kernel 3: merge a row's tile partials -> bf16 output columns (an empty
-// partial, l not above 0, weighs nothing)
+// partial, l 0, weighs nothing; a NaN one makes the row NaN)
 // ---------------------------------------------------------------------------
 struct MergeArgs {
   const float2* part_ml;  // (H*G, tile_stride): m, l
@@ -3271,10 +3271,11 @@ constexpr int kMergeFewParts = 128;
 
 // Merges N partials (m, l, acc), in order, into (mx, num, den): the running
 // sums are rescaled where a partial's m is above the maximum so far, else the
-// partial is; one that is empty (l not above 0) is skipped.  The maxima before
-// each partial, and so the weights, do not depend on the sums: only a multiply
-// and an add per partial are in the chain.  (A skipped partial adds -0, which
-// leaves any sum as it is.)
+// partial is.  An empty partial (l not above 0) is skipped; one whose l is NaN
+// (a NaN logit, which a maximum ignores) is not, and makes the sums NaN.  The
+// maxima before each partial, and so the weights, do not depend on the sums:
+// only a multiply and an add per partial are in the chain.  (A skipped partial
+// adds -0, which leaves any sum as it is.)
 template <int N>
 __device__ __forceinline__ void merge_fold(const float (&m)[N], const float (&l)[N],
                                            const float (&acc)[N], float& mx, float& num,
@@ -3283,7 +3284,7 @@ __device__ __forceinline__ void merge_fold(const float (&m)[N], const float (&l)
   bool up[N];
 #pragma unroll
   for (int u = 0; u < N; ++u) {
-    const bool live = l[u] > 0.0f;
+    const bool live = !(l[u] <= 0.0f);
     const float d = live ? m[u] - mx : 0.0f;
     lv[u] = live ? l[u] : -0.0f;
     av[u] = live ? acc[u] : -0.0f;
@@ -3363,7 +3364,7 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(MergeArgs a) {
 #pragma unroll
   for (int j = 0; j < kMergeK; ++j) x[j] = sn[j][tid < kMergeD ? tid : kMergeD];
   const int js = tid < kMergeK ? tid : kMergeK - 1;
-  const bool live = tid < kMergeK && sn[js][kMergeD] > 0.0f;
+  const bool live = tid < kMergeK && !(sn[js][kMergeD] <= 0.0f);
   float top = live ? sm[js] : kNegInf;
   const float mine = top;
 #pragma unroll
@@ -3380,7 +3381,8 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(MergeArgs a) {
     sum = (ups >> j) & 1u ? sum * wj + x[j] : __builtin_fmaf(x[j], wj, sum);
   }
   const float total = readlane(sum, kMergeD);
-  if (tid < kMergeD && d < D) a.out[r * D + d] = bf16_rne(sum / fmaxf(total, 1e-30f));
+  if (tid < kMergeD && d < D)
+    a.out[r * D + d] = bf16_rne(sum / (total < 1e-30f ? 1e-30f : total));
 }
 
 // ---------------------------------------------------------------------------

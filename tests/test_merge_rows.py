@@ -79,3 +79,54 @@ def test_dense_splits_match_attention(hip, tokens):
     out = hip.dense_decode(query, keys, values, length=tokens, workspace={})
     logits = query[0].double() @ keys[0].double().T.contiguous() / math.sqrt(96)
     _check(out.view(4, 96), logits.softmax(-1) @ values[0].double())
+
+
+@pytest.mark.parametrize("path", ["split", "step"])
+@pytest.mark.parametrize("what", ["suffix key", "query", "every suffix key"])
+@pytest.mark.parametrize("dim", [128, 256])
+def test_nan_reaches_the_output(hip, path, what, dim):
+    """A row whose logits hold a NaN comes out NaN, as softmax gives it (its
+    partial is not an empty one), and no row of another head; with three
+    kernels no other row at all."""
+    from refinekv import RefineKVConfig, build_summary, sparse_attention
+
+    gen = torch.Generator("cuda").manual_seed(dim)
+    rand = lambda *s: torch.randn(s, generator=gen, device="cuda").bfloat16()  # noqa: E731
+    heads, group, tokens, suffix = 2, 3, 1000, 33
+    query = rand(heads, group, 1, dim)
+    keys, values = rand(heads, tokens + suffix, dim), rand(heads, tokens + suffix, dim)
+    nan = torch.zeros(heads, group, dtype=torch.bool, device="cuda")
+    config = RefineKVConfig(backend="hip", eps=0.05)
+    summary = build_summary(keys[:, :tokens], values[:, :tokens], config)
+    if what == "query":
+        query[1, 2, 0, 5] = float("nan")
+        nan[1, 2] = True
+    else:
+        keys[1, tokens + 20 if what == "suffix key" else slice(tokens, None), 7] = float("nan")
+        nan[1] = True
+    hip.set_decode_path(path)
+    try:
+        out = sparse_attention(query, summary, keys[:, tokens:], values[:, tokens:],
+                               config).output
+    finally:
+        hip.set_decode_path("step")
+    got = out.isnan().view(heads, group, dim)
+    assert bool(got[nan].all()) and not bool(got[0].any())
+    if path == "split":
+        assert not bool(got[~nan].any())
+
+
+@pytest.mark.parametrize("what", ["key", "query", "every key"])
+def test_nan_reaches_the_dense_output(hip, what):
+    gen = torch.Generator("cuda").manual_seed(1)
+    rand = lambda *s: torch.randn(s, generator=gen, device="cuda").bfloat16()  # noqa: E731
+    query, keys, values = rand(2, 4, 64), rand(2, 5000, 64), rand(2, 5000, 64)
+    nan = torch.zeros(2, 4, dtype=torch.bool, device="cuda")
+    if what == "query":
+        query[1, 3, 9] = float("nan")
+        nan[1, 3] = True
+    else:
+        keys[0, 4321 if what == "key" else slice(None), 0] = float("nan")
+        nan[0] = True
+    out = hip.dense_decode(query, keys, values, workspace={})
+    assert torch.equal(out.isnan(), nan[..., None].expand(-1, -1, 64))
