@@ -21,7 +21,8 @@ CASES = [
     (2, 5, 96, 16, 1040, 17),
     (2, 2, 160, 32, 700, 6),       # two words per thread
     (2, 3, 256, 64, 999, 9),
-    (40, 4, 64, 16, 2100, 2),      # more (tile, head) cells than resident workgroups' rows
+    (40, 4, 64, 16, 2100, 2),      # many heads of few tiles
+    (2100, 1, 32, 16, 100, 9),     # more (tile, head) cells than resident workgroups
     (1, 4, 128, 16, 70000, 5),     # 69 tiles
 ]
 
