@@ -584,7 +584,10 @@ struct DecideArgs {
   const float* max_value_norm;  // (H)
   const uint8_t* anchor;        // (H, N) or null
   uint8_t* mask;                // (H, N)
-  bool write_mask;              // false: mask only stands in for a null anchor
+  // (always true; attend_tile_mma's mask store tests it all the same: without
+  // the test, however the branch was placed, the four-row step is 2 % slower,
+  // 8 layers at 131072 tokens 157 -> 160 us)
+  bool write_mask;
   float* risk_out;              // (H, G, N) or null
   float* stats_out;             // (H, G, 2) or null: log Z, log C
   const float* row_lse;         // (H, G, 2) log Z, log C merged once per row, or null
@@ -1046,7 +1049,7 @@ __device__ __forceinline__ uint64_t decide_finish(const DecideArgs& a, int64_t h
   }
   list = sh.list[wave];
   if (wave == 0) {
-    if (kMask && valid && owner && a.write_mask) a.mask[h * N + b] = sel ? 1 : 0;
+    if (kMask && valid && owner) a.mask[h * N + b] = sel ? 1 : 0;
     count = tile_access_count(a, tile, bits);
   }
   return bits;
@@ -2146,7 +2149,7 @@ __device__ void merge_slice(const AttendArgs& a, const StepCtx& sx, int64_t h, i
     }
   }
   RKV_STAMP(stamps, kStMergeStored, tid == 0);
-  if (poisoned && m == 0 && da.write_mask) {
+  if (poisoned && m == 0) {
     // (the workgroups' own mask stores wrote through before their partials,
     // so these come last)
     const int64_t N = da.n_blocks;
@@ -2255,8 +2258,8 @@ __device__ __forceinline__ void attend_tile(const AttendArgs& a, DecideShared& d
   // The launch's W workgroups per head: workgroup wk scores tile wk % T.
   // With short prompts the one-launch step runs copies of the T tiles (wk >=
   // T) so that the suffix and the head's expanded token rows spread over more
-  // workgroups: a copy repeats its tile's scores and decision (publishing the
-  // same slots, bit for bit) but adds no representatives of its own.
+  // workgroups: a copy repeats its tile's scores and decision but adds no
+  // representatives of its own.
   const uint32_t W = (uint32_t)a.workers;
   const uint32_t tile = wk % T;
   const bool primary = wk < T;
@@ -3082,11 +3085,11 @@ struct StepShared {
 #endif
 };
 
-// Workgroup (tile, h): the tile's scores (z, delta and the risk's delta
-// factors stay in LDS; the LSE partials are published and the head's
-// arrival counter bumped), then attend_tile's decision (after the head's
-// tiles have all arrived), attention and, for the head's last tile, the
-// merge.
+// Workgroup (w, h): the scores of tile w mod T (z, delta and the risk's delta
+// factors stay in LDS; the tile's first workgroup publishes its LSE partials
+// in tagged slots), then attend_tile_mma's decision (once the slots of all of
+// the head's tiles carry this launch's tag), its attention and, for the
+// head's last workgroups, a column slice of the merge.
 // kTicketed: (head, workgroup) from a start-order ticket instead of blockIdx
 // (grids larger than the device holds at once).
 // kTiles > 1: heads with more tiles than workgroups (W < n_tiles, four-row
@@ -3172,8 +3175,9 @@ void step_kernel(StepArgs s) {
   // a tile's LSE partials out as two tagged slots, by the tile's first
   // workgroup only: its copies hold the same, and 64 workgroups of a head of
   // one tile storing to the line they all poll made that wait 4.7 us (16 of
-  // each of four tiles 2.6; 64 tiles, no copies 1.5).  8 layers at 2048
-  // tokens 156 -> 126 us, at 8192 136 -> 130, group 7 at 8192 257 -> 182.
+  // each of four tiles 2.6; 64 tiles, no copies 1.5).  8 layers, 8 heads x 4
+  // rows: 2048 tokens 157 -> 127 us, 8192 139 -> 132; 4 x 7 at 8192 252 ->
+  // 173; 2 x 8 at 2048 384 -> 257, at 8192 319 -> 238.
   auto publish = [&](int64_t t, int g, float4 part) {
     if (kTiles == 1 && (uint32_t)wk >= (uint32_t)s.attend.decide.n_tiles) return;
     const uint32_t at = (uint32_t)(((h * G + g) * sa.tile_stride + t) * 2 * 16);
@@ -3266,7 +3270,11 @@ struct MergeArgs {
 // result (bf16 outputs change where fp32 sums are taken in another).
 // Latency bounds it: one round trip for a batch, then the fold.  The weights
 // of a batch are taken before its sums (merge_fold), so its exponentials do
-// not wait for one another, and the access count has a workgroup of its own.
+// not wait for one another, the stripes' weights are taken side by side, and
+// the access count has a workgroup of its own: 512 partials of 32 rows at
+// head_dim 128 8.5 -> 5.5 us (one weight after another, the stripes in one
+// lane, then the count, before; a lane tree in place of the order took 4.5),
+// the dense decode's 64 splits 4.6 -> 4.5.
 constexpr int kMergeFewParts = 128;
 
 // Merges N partials (m, l, acc), in order, into (mx, num, den): the running
@@ -3539,6 +3547,12 @@ int launch_select(const SelectParams& p, const Layout& L) {
 // one and a half for the summary rows it waits for; of the ways to cut a
 // head's rows the one whose rounds of workgroups cost least (more, shorter
 // workgroups fill the last round; fewer load the tile's summaries less often).
+// Whole calls, the chosen cut against the best of 1 to 64: 16 tiles, 32
+// anchors x 4 rows x 8 heads 25.8 / 25.2 us, 64 x 7 x 4 40.1 / 38.4, d 256 32 x
+// 8 x 2 24.9 / 25.3; 2 tiles, 64 x 4 x 8 11.0 / 11.0; 32 tiles, 64 x 6 x 2 35.4
+// / 34.2; 64 tiles, 16 x 4 x 8 46.9 / 42.1, 64 x 4 x 8 152.8 / 135.6 (there, of
+// many rounds, the last one overlaps the next workgroups' loads and counting it
+// whole is too dear); uncut they take 2 to 20 times as long.
 template <int D>
 int64_t anchor_slots() {
   static std::atomic<int> of_dev[64];  // per device; 0 = not asked yet
@@ -3557,10 +3571,20 @@ int64_t anchor_slots() {
   }
   return n;
 }
-constexpr int64_t kAnchorDecides = 2048;  // workgroups anchor_decide_kernel is cut into
+// Workgroups anchor_decide_kernel is cut into: below 1024 the decisions wait
+// for too few waves, above it nothing changes (whole calls at 256 / 512 / 1024
+// / 2048 / 8192: 32 anchors x 4 rows x 8 heads, 16 tiles 28.4 / 26.3 / 25.7 /
+// 25.8 / 25.7 us; 64 x 7 x 4, 16 tiles 42.4 / 40.4 / 40.0 / 40.0 / 39.9; 64 x
+// 1 x 8, 64 tiles, d 64 38.8 / 38.9 / 37.1 / 36.6 / 38.2).
+constexpr int64_t kAnchorDecides = 2048;
 // (row, tile) pairs up to which the decisions merge the rows' log Z / log C
-// themselves: a merge per pair instead of one per row, but one launch less
-// (16384 pairs: 7.1 us in one launch, 4.1 + 3.8 in two; 28672: 9.7 either way).
+// themselves: a merge per pair instead of one per row, but one launch less.
+// Whole calls, in one launch / in two: 8 heads x 4 rows, 16 tiles, 4096 pairs
+// 11.3 / 12.6 us, 12288 21.3 / 21.6, 16384 25.7 / 26.0, 24576 35.6 / 35.3,
+// 32768 46.5 / 45.4; 64 tiles, 8192 15.8 / 16.4, 16384 27.4 / 27.0, 32768 48.4
+// / 47.4; 4 x 7, 16 tiles, 14336 25.7 / 25.7, 28672 41.4 / 39.9; 8 x 1, 64
+// tiles, d 64, 16384 22.4 / 22.4, 32768 38.3 / 36.5: they cross between 14000
+// and 22000 pairs.
 constexpr int64_t kAnchorMerges = 20000;
 
 int launch_select_anchors(const SelectParams& p, int64_t anchors, int64_t q_as, int64_t q_hs,

@@ -1107,8 +1107,8 @@ extern "C" int rkv_summary_store(const void* keys, int64_t k_head_stride,
   return summary_impl("rkv_summary_store", keys, k_head_stride, k_token_stride, values,
                       v_head_stride, v_token_stride, dtype, heads, length, dim, block_size,
                       cache_keys, ck_head_stride, ck_token_stride, cache_values, cv_head_stride,
-                      cv_token_stride, nullptr, nullptr, counts, key_mean, value_mean, ellipsoid, value_norm,
-                      max_value_norm, stream);
+                      cv_token_stride, nullptr, nullptr, counts, key_mean, value_mean,
+                      ellipsoid, value_norm, max_value_norm, stream);
 }
 
 extern "C" int rkv_summary_pages(const void* keys, int64_t k_head_stride,

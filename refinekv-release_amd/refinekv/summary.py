@@ -145,8 +145,8 @@ def store_and_build_summary(keys: torch.Tensor, values: torch.Tensor, cache_keys
         fields = _hip.summary_fields(keys.detach(), values.detach(), block, cache_keys,
                                      cache_values, fill_keys, fill_values)
         counts, key_mean, value_mean, ellipsoid, value_norm, max_value_norm = fields
-        return BlockSummary(keys=key_pages, values=value_pages, counts=counts, key_mean=key_mean, value_mean=value_mean,
-                            ellipsoid=ellipsoid, value_norm=value_norm,
+        return BlockSummary(keys=key_pages, values=value_pages, counts=counts, key_mean=key_mean,
+                            value_mean=value_mean, ellipsoid=ellipsoid, value_norm=value_norm,
                             max_value_norm=max_value_norm, prompt_length=keys.shape[1],
                             block_size=block)
     cache_keys.copy_(keys)
