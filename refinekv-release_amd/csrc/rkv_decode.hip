@@ -4117,12 +4117,6 @@ extern "C" int rkv_select_anchors_strided(
     return set_error(kInvalidArgument, "%s: anchors must be in 1..65535", who);
   if (heads > 0 && heads * anchors > 65535)
     return set_error(kUnsupported, "%s: heads x anchors exceeds 65535", who);
-  // (an axis of length one has no stride: a tensor may carry any value there)
-  if (anchors == 1) q_anchor_stride = heads * group * dim;
-  if (heads == 1) q_head_stride = group * dim;
-  if (group == 1) q_row_stride = dim;
-  if (q_anchor_stride % 8 || q_head_stride % 8 || q_row_stride % 8)
-    return set_error(kInvalidArgument, "%s: query strides must be multiples of 8 elements", who);
   SelectParams p{queries, key_mean, ellipsoid, value_norm, max_value_norm, heads, group, dim,
                  n_blocks, block_size, prompt_length, eps, reduction, nullptr, mask_out,
                  nullptr, nullptr, nullptr, workspace, workspace_bytes, stream};
@@ -4133,6 +4127,12 @@ extern "C" int rkv_select_anchors_strided(
   if (workspace_bytes < (size_t)LA.total)
     return set_error(kWorkspaceTooSmall, "%s: workspace needs %lld bytes (rkv_workspace_bytes of "
                      "heads x anchors heads)", who, (long long)LA.total);
+  // (an axis of length one has no stride: a tensor may carry any value there)
+  if (anchors == 1) q_anchor_stride = heads * group * dim;
+  if (heads == 1) q_head_stride = group * dim;
+  if (group == 1) q_row_stride = dim;
+  if (q_anchor_stride % 8 || q_head_stride % 8 || q_row_stride % 8)
+    return set_error(kInvalidArgument, "%s: query strides must be multiples of 8 elements", who);
   return launch_select_anchors(p, anchors, q_anchor_stride, q_head_stride, q_row_stride);
 }
 

@@ -114,3 +114,25 @@ def test_workspace_size_covers_layout(lib):
         assert layout["step_workers"] == (want if several else max(tiles, want))
         assert tiles <= ts and layout["step_workers"] <= ts
     assert _hip.workspace_bytes(0, 4, 128, 10) == 0
+
+
+@pytest.mark.parametrize("change,code,text", [
+    (dict(dim=100), 2, b"head_dim 100"), (dict(dim=36), 2, b"head_dim 36"),
+    (dict(group=0), 1, b"shape"), (dict(group=17), 2, b"group 17"),
+    (dict(anchors=0), 1, b"anchors"), (dict(anchors=9000), 2, b"exceeds 65535"),
+    (dict(block=20), 1, b"block_size"), (dict(queries=None), 1, b"null"),
+    (dict(nbytes=100), 4, b"workspace"),
+])
+def test_anchor_selection_reports_what_is_wrong(lib, change, code, text):
+    """Bad arguments come back with the code of what is wrong with them, the
+    shape's before the strides that follow from it (host-side only: every call
+    here is refused before a launch)."""
+    raw = ctypes.create_string_buffer(4096)
+    at = ctypes.c_void_p(-(-ctypes.addressof(raw) // 256) * 256)
+    a = dict(queries=at, heads=8, group=4, dim=128, n_blocks=2, block=32, length=64, anchors=2,
+             nbytes=1 << 20)
+    a.update(change)
+    got = lib.rkv_select_anchors(a["queries"], at, at, at, at, a["heads"], a["group"], a["dim"],
+                                 a["n_blocks"], a["block"], a["length"], 0.01, 2, a["anchors"],
+                                 at, at, a["nbytes"], None)
+    assert got == code and text in lib.rkv_last_error(), lib.rkv_last_error()
