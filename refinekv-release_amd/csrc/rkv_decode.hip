@@ -4,8 +4,8 @@
 //
 // A decode step runs as ONE launch where the shape allows it (step_kernel):
 // workgroup (w, h) of the W per KV head h scores tile w mod T (64 blocks),
-// publishes its log-sum-exp partials in tagged slots, reads the head's T
-// tiles' slots, decides its blocks (risk, GQA reduction, anchors), folds its
+// publishes its log-sum-exp partials in tagged slots (a tile's first
+// workgroup does), reads the head's T tiles' slots, decides its blocks (risk, GQA reduction, anchors), folds its
 // representatives, its slice of the suffix and the token rows of its own
 // tile's expanded blocks (a copy of a tile, with more workgroups than
 // tiles, an even slice of them), publishes an (m, l, acc) partial in tagged
