@@ -5,14 +5,14 @@
 // A decode step runs as ONE launch where the shape allows it (step_kernel):
 // workgroup (w, h) of the W per KV head h scores tile w mod T (64 blocks),
 // publishes its log-sum-exp partials in tagged slots (a tile's first
-// workgroup does), reads the head's T tiles' slots, decides its blocks (risk, GQA reduction, anchors), folds its
-// representatives, its slice of the suffix and the token rows of its own
-// tile's expanded blocks (a copy of a tile, with more workgroups than
-// tiles, an even slice of them), publishes an (m, l, acc) partial in tagged
-// slots, and the head's last max(8, W / 4) workgroups by index (at most
-// head_dim / 2) each merge a column slice of the partials into the bf16
-// output.  Heads with more tiles
-// than workgroups score up to 4 tiles per workgroup in the same launch.
+// workgroup does), reads the head's T tiles' slots, decides its blocks (risk,
+// GQA reduction, anchors), folds its representatives, its slice of the suffix
+// and the token rows of its own tile's expanded blocks (a copy of a tile, with
+// more workgroups than tiles, an even slice of them), publishes an (m, l, acc)
+// partial in tagged slots, and the head's last max(8, W / 4) workgroups by
+// index (at most head_dim / 2) each merge a column slice of the partials into
+// the bf16 output.  Heads with more tiles than workgroups score up to 4 tiles
+// per workgroup in the same launch.
 // Other shapes run three kernels over the same workspace:
 //
 //   score  (tile, h)    one 64-block tile of head h: for every query row the
